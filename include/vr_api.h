@@ -134,7 +134,8 @@ typedef struct vr_ctx vr_ctx;
 void vr_default_config(vr_config* cfg, uint32_t width, uint32_t height);
 
 /* Create a render context on the current HIP device: allocates the top grid
- * (8 MiB), uber grid, brick pool (brick_capacity * 2 KiB), two hit buffers
+ * (8 MiB and a copy in the walk's order), uber grid, brick pool
+ * (brick_capacity * 2 KiB and 4 bytes per brick), two hit buffers
  * (12 B/px each), two reservoir buffers (36 B/px each) and the frame (16 B/px).
  * Replaces World::World's buffer set-up (template/world.cpp:47-193). */
 int vr_create(const vr_config* cfg, vr_ctx** out);
@@ -233,10 +234,10 @@ int vr_set_stage_waves(vr_ctx* ctx, int32_t stage, uint32_t waves);
 
 /* Traversal of the shadow rays of stage VR_STAGE_INITIAL or
  * VR_STAGE_RESOLVE (-1: both; the primary stage's rays always take the
- * nested DDA) for the following frames: VR_DDA_SCHEDULED (the default) runs
- * each turn of a wave's loop at the DDA level most of its lanes are at,
+ * nested DDA) for the following frames: VR_DDA_SCHEDULED (the default)
+ * steps the lanes of a wave together whatever DDA level each is at,
  * VR_DDA_NESTED walks the uber, top-grid and brick levels as nested loops,
- * which is faster where a wave's rays stay coherent.  A performance setting
+ * which can be faster where a wave's rays stay coherent.  A performance setting
  * with no counterpart in the reference (outputs are identical). */
 #define VR_DDA_SCHEDULED 0u
 #define VR_DDA_NESTED    1u

@@ -21,7 +21,30 @@ struct WorldView {
     const uint32_t* __restrict__ grid;    // [128^3] cell: 0 empty, c<<1 solid, id<<1|1 brick
     const uint32_t* __restrict__ bricks;  // pool [id*512 + lx + ly*8 + lz*64]
     const uint32_t* __restrict__ uber;    // [32^3 bits] cell x + z*32 + y*1024: some of its 4^3 cells non-empty
+    // the unified walk's copy of both grids (Walk below): it lies behind the
+    // pool in one allocation, so a 32-bit word index from `bricks` reaches
+    // every cell and voxel
+    const uint32_t* __restrict__ proj;    // [pool bricks] occupied slabs of a brick (brick_slabs)
+    uint32_t top;                         // word index of the first top-grid cell (kTopWords, then kUberWords)
 };
+
+// The copy's cells are stored so that the walk indexes all three levels
+// alike, with s bits per axis inside a block: word (z << 2s) + (y << s) + x.
+//   uber cells   one block of s = 5
+//   top cells    a block of s = 2 per uber cell (blocks in uber-cell order)
+//   voxels       a block of s = 3 per brick (the pool's own layout)
+// Bit 31 of a cell marks a child block: an uber cell with a non-empty top
+// cell, or a brick (bits 0-21 its id); other top cells hold their colour
+// word, empty ones 0.
+constexpr uint32_t kTopWords = 128u * 128u * 128u, kUberWords = 32u * 32u * 32u;
+constexpr uint32_t kChild = 1u << 31;
+
+// Bits of a non-empty voxel (x, y, z) in its brick's `proj` word: the slabs
+// of its x, y and z (bits 0-7, 8-15, 16-23)
+__device__ __forceinline__ uint32_t brick_slabs(uint32_t x, uint32_t y, uint32_t z)
+{
+    return (1u << x) | (256u << y) | (65536u << z);
+}
 
 // Light record prepared by the host from struct Light (common.h:134-139):
 // a = (centre.xyz, size), b = (Le.rgb, position bits).  Le is
@@ -310,204 +333,271 @@ __device__ uint32_t trace(const WorldView& w, f3 A, f3 B, int steps, uint32_t th
     return 0u;
 }
 
-// voxel lx + 8 ly + 64 lz of a brick from a packed in-brick position
-// (lx << 20 | ly << 10 | lz, each 0..7): the three fields land on disjoint
-// bits, so a field extract and two shift-ors build the index
-__device__ __forceinline__ uint32_t brick_voxel(uint32_t p)
+// ---------------------------------------------------------------------------
+// The same traversal for rays that go their own ways, as shadow rays do.
+// trace() nests the brick walk inside the top-grid loop inside the uber
+// loop, so a wave runs each brick walk while the lanes that are not inside
+// a brick wait.  Stepping is the same arithmetic at every level, though: the
+// nearest of three crossing distances, one cell along its axis.  Here a lane
+// keeps the state of the level it is at in one set of registers, and a wave
+// runs one of two units per turn:
+//   step    every lane that has a cell to visit visits it (budget, solid
+//           cell or voxel, child block) and steps, whatever its level
+//   change  the lanes that left a block go back to its parent's state, and
+//           those that found a child block go into it
+// chosen by how many lanes wait for each (ballot counts, a scalar branch).
+// Every lane performs trace()'s operations in its order, so hits, distances
+// and sides are the same bits; what differs is which lanes run together.
+// The waves' issue slots are what bounds it.  Against the walk that ran one
+// of the three levels per turn (a wave of 64 shadow rays on c2's frames:
+// 288 turns, 8-14 lanes busy in each; here 141), whole frames at 1920x1080:
+// 2.48 -> 1.99 ms (c2, uniform lights), 2.29 -> 1.71 ms (letters at
+// 1600x1024, where trace() had been the faster of the two), 3.48 -> 2.40 ms
+// (many-light world at 1279x717, MIS merge).
+//
+// Brick walks that cannot hit are left out.  A walk that leaves its brick
+// without a hit changes nothing but `t` and `last`, which the parent's step
+// sets again.  The walk stays inside the box between the voxel it enters and
+// the point where the ray leaves the top cell, so if the brick has no
+// occupied slab in that box's range along some axis, the walk cannot hit.
+// The exit point is taken kSlack voxels further along the ray than
+// computed: inside the map (coordinates up to 2^10) positions and crossings
+// are off by less than 2^-8 voxels (rounding of A + V t and of at most 24
+// additions of |1/V|).  Rays whose coordinates are not within 2^20 walk
+// every brick (`solid` below).  On c2's frames 2.2 of a shadow ray's 3.9
+// brick walks are left out, 14 of its 25 voxel steps.
+constexpr float kSlack = 0.0625f;
+
+__device__ __forceinline__ uint32_t lanes(uint64_t mask) { return (uint32_t)__builtin_popcountll(mask); }
+
+// Parent levels' state of the workgroup's lanes (256 threads at most): the
+// uber cell's and the top cell's crossing distances and packed cell, and the
+// top block's first word.  In LDS, so that the walk fits the registers of
+// the kernels that trace.
+struct WalkLds {
+    float tx[2][256], ty[2][256], tz[2][256];
+    uint32_t p[2][256], base[256];
+};
+
+__device__ __forceinline__ WalkLds& walk_lds()
 {
-    return (p >> 20) | (__builtin_amdgcn_ubfe(p, 10u, 3u) << 3) | ((p & 7u) << 6);
+    __shared__ WalkLds l;
+    return l;
 }
 
-// TraceOpaqueRay (trace.cl:205-282) for rays that go their own ways, as
-// shadow rays do.  trace() nests the brick walk inside the top-grid loop
-// inside the uber loop, so a wave runs each brick walk while the lanes that
-// are not inside a brick wait (on c2's shadow rays about 4 of 64 lanes take
-// each brick step).  Here the same traversal is cut into units - one visit
-// and step of an uber cell, of a top cell, or of a voxel - and each turn of
-// the wave's loop runs the unit of one level, chosen from how many of the
-// wave's lanes are at each (ballot counts, so the choice is a scalar
-// branch); the other lanes keep their state.  Every lane performs the operations
-// of trace() in the same order (each level keeps its own tm registers, which
-// trace() saves and restores around a descent), so the results are the same
-// bits.  `resume`: the lane's next unit at its level is the step that
-// follows a child level's exit (trace() steps the parent right after the
-// child loop ends).  While its steps advance a coordinate, a brick walk
-// leaves its brick within 22 steps (7 per axis and the one that leaves), so
-// trace()'s cap of 24 steps per brick never ends it; a ray whose steps do
-// not advance (a NaN direction: a shadow ray gets one only when its sample
-// point is the shading point itself) is ended by that cap and the step
-// budget, and kCap keeps the cap (see trace_sched below).
-template <bool kCap>
-__device__ uint32_t trace_sched_walk(const WorldView& w, f3 A, f3 B, int steps, float& dist, uint32_t& side)
-{
-    if (fabsf(B.x) < 1e-8f) B.x = B.x < 0 ? -1e-8f : 1e-8f;
-    if (fabsf(B.y) < 1e-8f) B.y = B.y < 0 ? -1e-8f : 1e-8f;
-    if (fabsf(B.z) < 1e-8f) B.z = B.z < 0 ? -1e-8f : 1e-8f;
-    const f3 V = B;
-    const f3 rV = f3{1.0f / V.x, 1.0f / V.y, 1.0f / V.z};
-    const uint32_t ox = V.x > 0 ? 1u : 0u, oy = V.y > 0 ? 1u : 0u, oz = V.z > 0 ? 1u : 0u;
-    const uint32_t dx = V.x > 0 ? (1u << 20) : (0xfffu << 20);
-    const uint32_t dy = V.y > 0 ? (1u << 10) : 0xfffffc00u;
-    const uint32_t dz = V.z > 0 ? 1u : 0xffffffffu;
-    const f3 td = f3{fabsf(rV.x), fabsf(rV.y), fabsf(rV.z)};
-    float to = 0.0f;
-    uint32_t last = 0;
-    bool active = true;
-    if (A.x < 0 || A.y < 0 || A.z < 0 || A.x > 1024.0f || A.y > 1024.0f || A.z > 1024.0f) {
-        const float tx1 = -A.x * rV.x, tx2 = (1024.0f - A.x) * rV.x;
-        float tmin = fminf(tx1, tx2), tmax = fmaxf(tx1, tx2);
-        const float ty1 = -A.y * rV.y, ty2 = (1024.0f - A.y) * rV.y;
-        tmin = fmaxf(tmin, fminf(ty1, ty2)), tmax = fminf(tmax, fmaxf(ty1, ty2));
-        const float tz1 = -A.z * rV.z, tz2 = (1024.0f - A.z) * rV.z;
-        tmin = fmaxf(tmin, fminf(tz1, tz2)), tmax = fminf(tmax, fmaxf(tz1, tz2));
-        if (tmax < tmin || tmax <= 0) active = false;
-        A.x += tmin * V.x, A.y += tmin * V.y, A.z += tmin * V.z;
-        to = tmin;
-        if (A.y < 0.01f || A.y > (1024.0f - 1.01f)) last = 1;
-        if (A.z < 0.01f || A.z > (1024.0f - 1.01f)) last = 2;
+// what a lane does next: visit and step, nothing (its ray ended, or it has
+// none), or change its level
+enum WalkMode : uint32_t { kStep = 0u, kMiss = 1u, kHit = 2u, kIdle = 3u, kDown = 4u, kUp = 5u };
+
+template <int KIND>
+struct Walk {
+    // the ray: origin (inside the map, or moved to its border), direction,
+    // 1/direction, packed cell steps; distance to the moved origin
+    f3 A, V, rV;
+    uint32_t dx, dy, dz;
+    float to;
+    uint32_t solid;  // ~0: walk every brick
+    // the level the lane is at: crossing distances, packed cell inside the
+    // block, the block's first word and first cell, bits per axis, the bits
+    // that a cell outside the block has, the budget of a visit
+    float tx, ty, tz;
+    uint32_t p, base, org, s, outside;
+    int cost;
+    float t;
+    uint32_t last, o, mode;  // o: the current cell or voxel
+    int steps;
+
+    static constexpr uint32_t kOut5 = ~((31u << 20) | (31u << 10) | 31u);
+    static constexpr uint32_t kOut2 = ~((3u << 20) | (3u << 10) | 3u);
+    static constexpr uint32_t kOut3 = ~((7u << 20) | (7u << 10) | 7u);
+
+    // word of packed cell c of a block with b bits per axis
+    static __device__ __forceinline__ uint32_t cell(uint32_t c, uint32_t b)
+    {
+        return ((((c & 1023u) << b) + __builtin_amdgcn_ubfe(c, 10u, 10u)) << b) + (c >> 20);
     }
-    uint32_t up = (min(f2u(A.x) >> 5, 31u) << 20) + (min(f2u(A.y) >> 5, 31u) << 10) + min(f2u(A.z) >> 5, 31u);
-    // tm of the uber level (u*), of the top grid (g*) and of the brick (b*)
-    float ux = ((float)((up >> 20) + ox) - A.x * 0.03125f) * rV.x;
-    float uy = ((float)(((up >> 10) & 31u) + oy) - A.y * 0.03125f) * rV.y;
-    float uz = ((float)((up & 31u) + oz) - A.z * 0.03125f) * rV.z;
-    float gx = 0.0f, gy = 0.0f, gz = 0.0f, bx = 0.0f, by = 0.0f, bz = 0.0f;
-    float t = 0.0f;
-    uint32_t tp = 0u, p = 0u, brick = 0u;
-    // the lane's level: 0 uber, 1 top grid, 2 brick; 3 done without a hit,
-    // 4 hit a solid top-grid cell, 5 hit a voxel.  `resume` (see above) for
-    // the level it is at.  Inside a unit the lanes of that level update their
-    // state with selects (the other lanes keep theirs), so the loop has
-    // little control flow for the compiler to copy registers across.
-    uint32_t lv = active ? 0u : 3u, resume = 0u;
-    // the occupancy of the lane's current cell: uber bit, top-grid word or voxel
-    uint32_t o = active ? uber_bit(w.uber, (up >> 20) + ((up & 31u) << 5) + (((up >> 10) & 31u) << 10)) : 0u;
-    while (true) {
-        const uint32_t n0 = (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(lv == 0u));
-        const uint32_t n1 = (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(lv == 1u));
-        const uint32_t n2 = (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(lv == 2u));
-        if ((n0 | n1 | n2) == 0u) break;
-        // The level to run: bricks when at least half as many lanes are in
-        // a brick as at either other level, then the top grid when at least
-        // twice as many lanes are there as at the uber level, else the uber
-        // level (of the weightings tried on c2, the fastest: brick units are
-        // the cheapest, and running the uber level first gathers lanes into
-        // the top grid's more costly units)
-        if (2u * n2 >= n1 && 2u * n2 >= n0) {
-            // voxels of the brick walks, for as long as that holds (an inner
-            // loop: its state stays in place between turns)
-            uint32_t m1 = n1, m2 = n2;
-            do {
-                const bool mine = lv == 2u;
-                const bool stop = mine && (o & 0xf000u) == 0xf000u;
-                const bool go = mine && !stop;
-                const float tn = fminf(bx, fminf(by, bz));
-                const bool sx = go && tn == bx, sy = go && tn == by, sz = go && tn == bz;
-                bx = sx ? bx + td.x : bx;
-                by = sy ? by + td.y : by;
-                bz = sz ? bz + td.z : bz;
-                p += (sx ? dx : 0u) + (sy ? dy : 0u) + (sz ? dz : 0u);
-                last = go ? (sz ? 2u : (sy ? 1u : 0u)) : last;
-                t = go ? tn : t;
-                const bool out = go && ((p & kTopMask3) != 0u || (kCap && resume == 23u));
-                lv = stop ? 5u : (out ? 1u : lv);
-                resume = out ? 1u : (kCap && go ? resume + 1u : resume);
-                if (go && !out) o = w.bricks[(size_t)brick * 512u + brick_voxel(p)];
-                m1 = (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(lv == 1u));
-                m2 = (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(lv == 2u));
-            } while (2u * m2 >= m1 && 2u * m2 >= n0 && m2 != 0u);
-        } else if (n1 >= 2u * n0) {
-            // a cell of the top grid: visit (budget, solid cell, brick), then
-            // step unless the lane stopped or went into a brick
-            const bool mine = lv == 1u;
-            const bool visit = mine && resume == 0u;
-            steps = visit ? steps - 1 : steps;
-            const bool spent = visit && steps == 0;
-            const bool solid = visit && !spent && (o & 1u) == 0u;
-            const bool stop = solid && ((o >> 1) & 0xf000u) == 0xf000u;
-            const bool down = visit && !spent && (o & 1u) != 0u;
-            if (down) {
-                t *= 8.0f;
-                const uint32_t q4x = f2u(A.x + V.x * t);
-                const uint32_t q4y = f2u(A.y + V.y * t);
-                const uint32_t q4z = f2u(A.z + V.z * t);
-                const uint32_t cx8 = (tp >> 20) << 3, cy8 = ((tp >> 10) & 127u) << 3, cz8 = (tp & 127u) << 3;
-                p = (clampu(q4x, cx8, cx8 + 7) << 20) + (clampu(q4y, cy8, cy8 + 7) << 10) + clampu(q4z, cz8, cz8 + 7);
-                bx = ((float)((p >> 20) + ox) - A.x) * rV.x;
-                by = ((float)(((p >> 10) & 1023u) + oy) - A.y) * rV.y;
-                bz = ((float)((p & 1023u) + oz) - A.z) * rV.z;
-                p &= 7u + (7u << 10) + (7u << 20);
-                brick = o >> 1;
-                o = w.bricks[(size_t)brick * 512u + brick_voxel(p)];
-            }
-            const bool go = mine && !spent && !stop && !down;
-            const float tn = fminf(gx, fminf(gy, gz));
-            const bool sx = go && tn == gx, sy = go && tn == gy, sz = go && tn == gz;
-            gx = sx ? gx + td.x : gx;
-            gy = sy ? gy + td.y : gy;
-            gz = sz ? gz + td.z : gz;
-            tp += (sx ? dx : 0u) + (sy ? dy : 0u) + (sz ? dz : 0u);
-            last = go ? (sz ? 2u : (sy ? 1u : 0u)) : last;
-            t = go ? tn : t;
-            const bool out = go && (tp & kUberMask3) != (up << 2);
-            lv = stop ? 4u : (down ? 2u : ((spent || out) ? 0u : lv));
-            resume = (spent || out) ? 1u : (mine ? 0u : resume);
-            if (go && !out) o = w.grid[(tp >> 20) + ((tp & 127u) << 7) + (((tp >> 10) & 127u) << 14)];
-        } else {
-            // a cell of the uber grid: visit (budget, occupied cell), then
-            // step unless the lane stopped or went into the top grid
-            const bool mine = lv == 0u;
-            const bool visit = mine && resume == 0u;
-            steps = visit ? steps - 4 : steps;
-            const bool spent = visit && steps <= 0;
-            const bool down = visit && !spent && o != 0u;
-            if (down) {
-                t *= 4.0f;
-                const uint32_t p4x = f2u(0.125f * A.x + V.x * t);
-                const uint32_t p4y = f2u(0.125f * A.y + V.y * t);
-                const uint32_t p4z = f2u(0.125f * A.z + V.z * t);
-                const uint32_t bx4 = (up >> 20) << 2, by4 = ((up >> 10) & 31u) << 2, bz4 = (up & 31u) << 2;
-                tp = (clampu(p4x, bx4, bx4 + 3) << 20) + (clampu(p4y, by4, by4 + 3) << 10) + clampu(p4z, bz4, bz4 + 3);
-                gx = ((float)((tp >> 20) + ox) - A.x * 0.125f) * rV.x;
-                gy = ((float)(((tp >> 10) & 127u) + oy) - A.y * 0.125f) * rV.y;
-                gz = ((float)((tp & 127u) + oz) - A.z * 0.125f) * rV.z;
-                o = w.grid[(tp >> 20) + ((tp & 127u) << 7) + (((tp >> 10) & 127u) << 14)];
-            }
-            const bool go = mine && !spent && !down;
-            const float tn = fminf(ux, fminf(uy, uz));
-            const bool sx = go && tn == ux, sy = go && tn == uy, sz = go && tn == uz;
-            ux = sx ? ux + td.x : ux;
-            uy = sy ? uy + td.y : uy;
-            uz = sz ? uz + td.z : uz;
-            up += (sx ? dx : 0u) + (sy ? dy : 0u) + (sz ? dz : 0u);
-            last = go ? (sz ? 2u : (sy ? 1u : 0u)) : last;
-            t = go ? tn : t;
-            const bool out = go && (up & 0xfe0f83e0u) != 0u;
-            lv = (spent || out) ? 3u : (down ? 1u : lv);
-            resume = mine ? 0u : resume;
-            if (go && !out) o = uber_bit(w.uber, (up >> 20) + ((up & 31u) << 5) + (((up >> 10) & 31u) << 10));
+
+    // the ray's first cell; trace()'s set-up
+    __device__ __forceinline__ void begin(const WorldView& w, f3 A0, f3 B, int budget)
+    {
+        constexpr float kBound = 1048576.0f;
+        const bool bounded = fabsf(A0.x) <= kBound && fabsf(A0.y) <= kBound && fabsf(A0.z) <= kBound &&
+                             fabsf(B.x) <= kBound && fabsf(B.y) <= kBound && fabsf(B.z) <= kBound;
+        solid = bounded ? 0u : ~0u;
+        if (fabsf(B.x) < 1e-8f) B.x = B.x < 0 ? -1e-8f : 1e-8f;
+        if (fabsf(B.y) < 1e-8f) B.y = B.y < 0 ? -1e-8f : 1e-8f;
+        if (fabsf(B.z) < 1e-8f) B.z = B.z < 0 ? -1e-8f : 1e-8f;
+        A = A0, V = B;
+        rV = f3{1.0f / V.x, 1.0f / V.y, 1.0f / V.z};
+        dx = V.x > 0 ? (1u << 20) : (0xfffu << 20);
+        dy = V.y > 0 ? (1u << 10) : 0xfffffc00u;
+        dz = V.z > 0 ? 1u : 0xffffffffu;
+        to = 0.0f, t = 0.0f, last = 0u, steps = budget, mode = kStep;
+        if (A.x < 0 || A.y < 0 || A.z < 0 || A.x > 1024.0f || A.y > 1024.0f || A.z > 1024.0f) {
+            const float tx1 = -A.x * rV.x, tx2 = (1024.0f - A.x) * rV.x;
+            float tmin = fminf(tx1, tx2), tmax = fmaxf(tx1, tx2);
+            const float ty1 = -A.y * rV.y, ty2 = (1024.0f - A.y) * rV.y;
+            tmin = fmaxf(tmin, fminf(ty1, ty2)), tmax = fminf(tmax, fmaxf(ty1, ty2));
+            const float tz1 = -A.z * rV.z, tz2 = (1024.0f - A.z) * rV.z;
+            tmin = fmaxf(tmin, fminf(tz1, tz2)), tmax = fminf(tmax, fmaxf(tz1, tz2));
+            if (tmax < tmin || tmax <= 0) mode = kMiss;
+            A.x += tmin * V.x, A.y += tmin * V.y, A.z += tmin * V.z;
+            to = tmin;
+            if (A.y < 0.01f || A.y > (1024.0f - 1.01f)) last = 1;
+            if (A.z < 0.01f || A.z > (1024.0f - 1.01f)) last = 2;
+        }
+        const uint32_t cx = min(f2u(A.x) >> 5, 31u), cy = min(f2u(A.y) >> 5, 31u), cz = min(f2u(A.z) >> 5, 31u);
+        p = (cx << 20) | (cy << 10) | cz;
+        tx = ((float)(cx + (V.x > 0 ? 1u : 0u)) - A.x * 0.03125f) * rV.x;
+        ty = ((float)(cy + (V.y > 0 ? 1u : 0u)) - A.y * 0.03125f) * rV.y;
+        tz = ((float)(cz + (V.z > 0 ? 1u : 0u)) - A.z * 0.03125f) * rV.z;
+        base = w.top + kTopWords, org = 0u, s = 5u, outside = kOut5, cost = 4;
+        o = w.bricks[(size_t)(base + cell(p, 5u))];
+    }
+
+    // Lanes in kStep: visit the cell, then step to the next one; the others
+    // keep their state (selects instead of branches: the compiler copies
+    // registers across divergent joins).
+    __device__ __forceinline__ void step(const WorldView& w)
+    {
+        const bool mine = mode == kStep;
+        steps -= mine ? cost : 0;
+        const bool child = (int32_t)o < 0 && s != 3u;
+        const bool stops = KIND == kTraceAll ? o != 0u : (o & 0xf000u) == 0xf000u;
+        const bool go = mine && steps > 0 && !child && !stops;
+        const float tn = fminf(tx, fminf(ty, tz));
+        const bool sx = go && tn == tx, sy = go && tn == ty, sz = go && tn == tz;
+        tx += sx ? fabsf(rV.x) : 0.0f;
+        ty += sy ? fabsf(rV.y) : 0.0f;
+        tz += sz ? fabsf(rV.z) : 0.0f;
+        p += (sx ? dx : 0u) + (sy ? dy : 0u) + (sz ? dz : 0u);
+        last = go ? (sz ? 2u : (sy ? 1u : 0u)) : last;
+        t = go ? tn : t;
+        const bool out = go && (p & outside) != 0u;
+        uint32_t next = child ? kDown : (stops ? kHit : kStep);
+        next = steps <= 0 || out ? (s == 5u ? kMiss : kUp) : next;
+        mode = mine ? next : mode;
+        if (go && !out) {
+            uint32_t at = base + cell(p, s);
+            asm volatile("; step" : "+v"(at));  // keeps the load in this unit
+            o = w.bricks[(size_t)at];
         }
     }
-    uint32_t hit = 0u;
-    if (lv == 5u) hit = o, dist = t + to, side = last;
-    if (lv == 4u) hit = o >> 1, dist = t * 8.0f + to, side = last;
-    return hit;
-}
 
-// With every coordinate of the origin and the direction within +-2^20 (so
-// finite: a NaN fails the comparisons), 2^-27 < |1/V| < 2^27 after
-// FixZeroDeltas, and every tm, t and position product of the walk stays
-// finite, so each step advances a coordinate.  A wave with a ray outside
-// those bounds (a NaN direction; vr_trace_rays refuses non-finite rays but
-// takes large ones) walks with trace()'s cap of 24 steps per brick, counted
-// in `resume`; other waves do not pay for the count.
-__device__ __forceinline__ uint32_t trace_sched(const WorldView& w, f3 A, f3 B, int steps, float& dist, uint32_t& side)
+    // Lanes in kUp: back to the parent, whose pending step follows without
+    // another visit (an empty cell, its budget given back)
+    __device__ __forceinline__ void up_level(const WorldView& w)
+    {
+        WalkLds& l = walk_lds();
+        const bool brick = s == 3u;
+        const int k = brick ? 1 : 0;
+        tx = l.tx[k][threadIdx.x], ty = l.ty[k][threadIdx.x], tz = l.tz[k][threadIdx.x], p = l.p[k][threadIdx.x];
+        base = brick ? l.base[threadIdx.x] : w.top + kTopWords;
+        org = (org >> s) - p;  // a block's first cell is its parent's cell << s
+        s = brick ? 2u : 5u, outside = brick ? kOut2 : kOut5, cost = brick ? 1 : 4;
+        steps += cost, o = 0u, mode = kStep;
+    }
+
+    // one axis of the box test: the brick's slabs between local cells a and b
+    static __device__ __forceinline__ uint32_t slabs_between(uint32_t slabs, uint32_t a, uint32_t b)
+    {
+        const uint32_t n = (a > b ? a - b : b - a) + 1u;
+        return slabs & (((1u << n) - 1u) << min(a, b));
+    }
+
+    static __device__ __forceinline__ uint32_t med3(uint32_t v, uint32_t lo, uint32_t hi) { return min(max(v, lo), hi); }
+
+    // lanes in kDown: into the child block of the current cell
+    __device__ __forceinline__ void down_level(const WorldView& w)
+    {
+        WalkLds& l = walk_lds();
+        const bool top = s == 2u;  // at the top grid: the child is a brick
+        uint32_t slabs = ~0u;
+        if (top) slabs = w.proj[o & 0x3fffffu] | solid;
+        const uint32_t bits = top ? 3u : 2u;
+        const float scale = top ? 1.0f : 0.125f;  // map -> child cells
+        const float grow = top ? 8.0f : 4.0f;     // child cells per cell
+        const f3 As = f3{A.x * scale, A.y * scale, A.z * scale};
+        const float tc = t * grow;
+        const uint32_t first = (org + p) << bits;  // the child block's first cell
+        const uint32_t lx = first >> 20, ly = __builtin_amdgcn_ubfe(first, 10u, 10u), lz = first & 1023u;
+        const uint32_t n1 = top ? 7u : 3u;
+        const uint32_t cx = med3(f2u(As.x + V.x * tc), lx, lx + n1);
+        const uint32_t cy = med3(f2u(As.y + V.y * tc), ly, ly + n1);
+        const uint32_t cz = med3(f2u(As.z + V.z * tc), lz, lz + n1);
+        const float te = fminf(tx, fminf(ty, tz)) * grow;
+        const uint32_t ex = med3(f2u(__builtin_fmaf(V.x, te, As.x + copysignf(kSlack, V.x))), lx, lx + n1);
+        const uint32_t ey = med3(f2u(__builtin_fmaf(V.y, te, As.y + copysignf(kSlack, V.y))), ly, ly + n1);
+        const uint32_t ez = med3(f2u(__builtin_fmaf(V.z, te, As.z + copysignf(kSlack, V.z))), lz, lz + n1);
+        const uint32_t bx = slabs_between(slabs & 255u, cx - lx, ex - lx);
+        const uint32_t by = slabs_between((slabs >> 8) & 255u, cy - ly, ey - ly);
+        const uint32_t bz = slabs_between((slabs >> 16) & 255u, cz - lz, ez - lz);
+        const bool may = min(min(bx, by), bz) != 0u;
+        // the parent's state (unused at a brick that is left out)
+        const int k = top ? 1 : 0;
+        l.tx[k][threadIdx.x] = tx, l.ty[k][threadIdx.x] = ty, l.tz[k][threadIdx.x] = tz, l.p[k][threadIdx.x] = p;
+        if (top) l.base[threadIdx.x] = base;
+        const uint32_t child = top ? o << 9 : w.top + (cell(p, 5u) << 6);
+        steps += may ? 0 : cost;
+        t = may ? tc : t;
+        tx = may ? ((float)(cx + (V.x > 0 ? 1u : 0u)) - As.x) * rV.x : tx;
+        ty = may ? ((float)(cy + (V.y > 0 ? 1u : 0u)) - As.y) * rV.y : ty;
+        tz = may ? ((float)(cz + (V.z > 0 ? 1u : 0u)) - As.z) * rV.z : tz;
+        p = may ? ((cx - lx) << 20) | ((cy - ly) << 10) | (cz - lz) : p;
+        base = may ? child : base;
+        org = may ? first : org;
+        s = may ? bits : s;
+        outside = may ? (top ? kOut3 : kOut2) : outside;
+        cost = may ? (top ? 0 : 1) : cost;
+        o = 0u;
+        if (may) o = w.bricks[(size_t)(base + cell(p, s))];
+        mode = kStep;
+    }
+
+    __device__ __forceinline__ float distance() const { return (s == 3u ? t : t * 8.0f) + to; }
+
+    __device__ __forceinline__ uint64_t stepping() const { return __builtin_amdgcn_ballot_w64(mode == kStep); }
+    __device__ __forceinline__ uint64_t changing() const { return __builtin_amdgcn_ballot_w64(mode > kIdle); }
+    __device__ __forceinline__ bool more_steps() const { return (int)lanes(stepping()) - (int)lanes(changing()) > 0; }
+
+    // Step turns while more lanes have a cell to visit than a level to change.
+    // A lane is in the brick it is in since before the run (only a change
+    // turn enters one), and a brick walk that advances leaves within 22 steps
+    // (7 per axis and the one that leaves).  A ray whose steps do not advance
+    // (a NaN direction: a shadow ray gets one only when its sample point is
+    // the shading point itself) would stay, so a run ends after 32 turns and
+    // the lanes still stepping inside a brick are sent up; the visits they
+    // repeated were of one voxel, as in trace()'s 24.
+    __device__ __forceinline__ void step_run(const WorldView& w)
+    {
+        uint32_t n = 0u;
+        if (more_steps()) do {
+            step(w);
+            n++;
+        } while (more_steps() && n < 32u);
+        if (n == 32u) mode = mode == kStep && s == 3u ? kUp : mode;
+    }
+
+    __device__ __forceinline__ void change(const WorldView& w)
+    {
+        if (mode == kUp) up_level(w);
+        if (mode == kDown) down_level(w);
+    }
+};
+
+template <int KIND>
+__device__ __forceinline__ uint32_t trace_free(const WorldView& w, f3 A, f3 B, int steps, float& dist, uint32_t& side)
 {
-    constexpr float kBound = 1048576.0f;
-    const bool bounded = fabsf(A.x) <= kBound && fabsf(A.y) <= kBound && fabsf(A.z) <= kBound &&
-                         fabsf(B.x) <= kBound && fabsf(B.y) <= kBound && fabsf(B.z) <= kBound;
-    if (__builtin_amdgcn_ballot_w64(!bounded) != 0u) return trace_sched_walk<true>(w, A, B, steps, dist, side);
-    return trace_sched_walk<false>(w, A, B, steps, dist, side);
+    Walk<KIND> k;
+    k.begin(w, A, B, steps);
+    while (true) {
+        k.step_run(w);
+        if ((k.stepping() | k.changing()) == 0u) break;
+        k.change(w);
+    }
+    if (k.mode != kHit) return 0u;
+    dist = k.distance(), side = k.last;
+    return k.o;
 }
 
 // ---------------------------------------------------------------------------

@@ -20,9 +20,10 @@ struct LightMotionView {
     uint32_t n;
 };
 
-hipError_t launch_edit_bricks(uint32_t* pool, uint32_t highWater, uint32_t frame, uint32_t seed, uint32_t permille,
-                              uint32_t steps, hipStream_t s);
-hipError_t launch_move_lights(const LightMotionView& m, const uint32_t* grid, uint32_t* pool, uint32_t cap,
-                              hipStream_t s);
+// proj: the bricks' occupied slabs (WorldView::proj), kept a superset
+hipError_t launch_edit_bricks(uint32_t* pool, uint32_t* proj, uint32_t highWater, uint32_t frame, uint32_t seed,
+                              uint32_t permille, uint32_t steps, hipStream_t s);
+hipError_t launch_move_lights(const LightMotionView& m, const uint32_t* grid, uint32_t* pool, uint32_t* proj,
+                              uint32_t cap, hipStream_t s);
 
 }  // namespace vr

@@ -24,9 +24,12 @@ __device__ __forceinline__ uint32_t edit_hash(uint32_t id, uint32_t frame, uint3
 // (opaque, no emission); each of `steps` steps draws r = xorshift(s), moves
 // one voxel along axis r % 3 (up if r >> 8 & 1, wrapping inside the brick)
 // and toggles the voxel it lands on between empty and the colour; emissive
-// voxels are left alone.  One lane per brick.
-__global__ __launch_bounds__(256) void k_edit_bricks(uint32_t* __restrict__ pool, uint32_t highWater, uint32_t frame,
-                                                     uint32_t seed, uint32_t permille, uint32_t steps)
+// voxels are left alone.  One lane per brick.  The brick's occupied slabs
+// only grow (an emptied voxel may leave its slabs marked, which costs a walk
+// that could have been left out and no correctness).
+__global__ __launch_bounds__(256) void k_edit_bricks(uint32_t* __restrict__ pool, uint32_t* __restrict__ proj,
+                                                     uint32_t highWater, uint32_t frame, uint32_t seed,
+                                                     uint32_t permille, uint32_t steps)
 {
     const uint32_t id = blockIdx.x * 256u + threadIdx.x;
     if (id >= highWater) return;
@@ -36,6 +39,7 @@ __global__ __launch_bounds__(256) void k_edit_bricks(uint32_t* __restrict__ pool
     uint32_t c[3] = {s & 7u, (s >> 3) & 7u, (s >> 6) & 7u};
     const uint32_t colour = 0xF000u | ((s >> 9) & 0xFFFu);
     uint32_t* b = pool + (size_t)id * 512u;
+    uint32_t slabs = 0u;
     for (uint32_t k = 0; k < steps; k++) {
         const uint32_t r = xorshift(s);
         const uint32_t axis = r % 3u;
@@ -47,7 +51,9 @@ __global__ __launch_bounds__(256) void k_edit_bricks(uint32_t* __restrict__ pool
         const uint32_t old = *v;
         if ((old >> 16) & 255u) continue;
         *v = old ? 0u : colour;
+        if (!old) slabs |= brick_slabs(c[0], c[1], c[2]);
     }
+    proj[id] |= slabs;
 }
 
 __global__ __launch_bounds__(256) void k_fill_u32(uint32_t* __restrict__ p, uint32_t n, uint32_t v)
@@ -118,7 +124,8 @@ __global__ __launch_bounds__(256) void k_light_claim(LightMotionView m, const ui
 // cleared, the light record (centre, packed position) updated; the losers
 // bounce.
 __global__ __launch_bounds__(256) void k_light_move(LightMotionView m, const uint32_t* __restrict__ grid,
-                                                    uint32_t* __restrict__ pool, uint32_t cap)
+                                                    uint32_t* __restrict__ pool, uint32_t* __restrict__ proj,
+                                                    uint32_t cap)
 {
     const uint32_t i = blockIdx.x * 256u + threadIdx.x;
     if (i >= m.n) return;
@@ -135,6 +142,7 @@ __global__ __launch_bounds__(256) void k_light_move(LightMotionView m, const uin
     (void)voxel_slot(grid, cap, tx, ty, tz, st);  // the claim checked it
     if (voxel_slot(grid, cap, cx, cy, cz, sc)) pool[sc] = 0u;
     pool[st] = m.voxel[i];
+    atomicOr(&proj[st >> 9], brick_slabs(tx & 7u, ty & 7u, tz & 7u));  // slabs only grow, as in k_edit_bricks
     const float4 p = m.pos[i], v = m.vel[i];
     m.pos[i] = make_float4(p.x + v.x, p.y + v.y, p.z + v.z, 0.0f);
     m.la[i] = make_float4((float)tx + 0.5f, (float)ty + 0.5f, (float)tz + 0.5f, 1.0f);
@@ -144,22 +152,22 @@ __global__ __launch_bounds__(256) void k_light_move(LightMotionView m, const uin
 
 }  // namespace
 
-hipError_t launch_edit_bricks(uint32_t* pool, uint32_t highWater, uint32_t frame, uint32_t seed, uint32_t permille,
+hipError_t launch_edit_bricks(uint32_t* pool, uint32_t* proj, uint32_t highWater, uint32_t frame, uint32_t seed, uint32_t permille,
                               uint32_t steps, hipStream_t s)
 {
     if (highWater == 0 || permille == 0 || steps == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_edit_bricks, dim3((highWater + 255) / 256), dim3(256), 0, s, pool, highWater, frame, seed,
+    hipLaunchKernelGGL(k_edit_bricks, dim3((highWater + 255) / 256), dim3(256), 0, s, pool, proj, highWater, frame, seed,
                        permille, steps);
     return hipGetLastError();
 }
 
-hipError_t launch_move_lights(const LightMotionView& m, const uint32_t* grid, uint32_t* pool, uint32_t cap,
-                              hipStream_t s)
+hipError_t launch_move_lights(const LightMotionView& m, const uint32_t* grid, uint32_t* pool, uint32_t* proj,
+                              uint32_t cap, hipStream_t s)
 {
     if (m.n == 0) return hipSuccess;
     hipLaunchKernelGGL(k_fill_u32, dim3(kClaimBuckets / 256), dim3(256), 0, s, m.claim, kClaimBuckets, kNoTarget);
     hipLaunchKernelGGL(k_light_claim, dim3((m.n + 255) / 256), dim3(256), 0, s, m, grid, pool, cap);
-    hipLaunchKernelGGL(k_light_move, dim3((m.n + 255) / 256), dim3(256), 0, s, m, grid, pool, cap);
+    hipLaunchKernelGGL(k_light_move, dim3((m.n + 255) / 256), dim3(256), 0, s, m, grid, pool, proj, cap);
     return hipGetLastError();
 }
 

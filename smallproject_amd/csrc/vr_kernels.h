@@ -115,7 +115,7 @@ __device__ __forceinline__ void tile_of_block(uint32_t order, int& tx, int& ty)
 }
 
 // traversal of a stage's shadow rays (FrameArgs::dda; the values of
-// VR_DDA_SCHEDULED and VR_DDA_NESTED): the wave-scheduled DDA, or the
+// VR_DDA_SCHEDULED and VR_DDA_NESTED): the wave-scheduled walk, or the
 // nested one of the primary rays
 constexpr uint32_t kDdaScheduled = 0u, kDdaNested = 1u;
 
@@ -150,7 +150,7 @@ struct MisBufs {
 // the list's capacity
 hipError_t launch_mis_split(const FrameArgs& a, const MisBufs& m, uint32_t traceBlocks, hipStream_t s);
 // Up to kChunkViews views rendered by one launch per stage: their
-// FrameArgs travel in the kernel argument (8 x 448 B + the tile table,
+// FrameArgs travel in the kernel argument (8 x 472 B + the tile table,
 // under the 4 KiB kernel-argument limit), so pointers in them are global
 // pointers to the compiler as in the one-view kernels.
 constexpr int kChunkViews = 8;
@@ -168,9 +168,10 @@ hipError_t launch_stage_views(int stage, const ViewChunk& c, uint32_t blocks, bo
 // pointer; c and args must stay valid while the node is added or updated)
 hipError_t stage_views_node(int stage, const ViewChunk* c, uint32_t blocks, bool anyMis, void** args,
                             hipKernelNodeParams* p);
-hipError_t launch_commit(const uint32_t* ids, const uint32_t* src, uint32_t* pool, uint32_t n, uint32_t cap,
-                         hipStream_t s);
-hipError_t launch_uber(const uint32_t* grid, uint32_t* uber, hipStream_t s);
+hipError_t launch_commit(const uint32_t* ids, const uint32_t* src, uint32_t* pool, uint32_t* proj, uint32_t n,
+                         uint32_t cap, hipStream_t s);
+// the uber bits and the unified walk's cells from the top grid
+hipError_t launch_uber(const uint32_t* grid, uint32_t* uber, uint32_t* cells, hipStream_t s);
 hipError_t launch_trace_batch(const WorldView& w, const float* O, const float* D, uint32_t n, uint32_t kind,
                               int32_t steps, uint32_t* voxel, float* dist, uint32_t* side, hipStream_t s);
 hipError_t launch_ground_truth(const FrameArgs& a, uint32_t spp, uint32_t frame0, double* accum, hipStream_t s);

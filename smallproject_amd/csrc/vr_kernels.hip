@@ -89,22 +89,16 @@ __device__ __forceinline__ void count_rays(unsigned long long* rays, int k, uint
 // GridCoordinatesFromHit + Uint3CubeEquals (cl/tools.cl:452-472) behind
 // isLightOccluded (cl/ris.cl:1-17).  A shadow ray that finds no opaque voxel
 // within its step budget counts as occluded.  Shadow rays of a wave head to
-// different lights, so they take the wave-scheduled DDA: kPick picks the
-// walk per wave (trace_sched: uncounted unless a ray is out of bounds), else
-// the walk that counts its brick steps runs always (one copy of the loop:
-// for the shading pass's rays a second copy costs more registers than the
-// count costs their fewer rays; the MIS merge's kernel, with more registers
-// per lane, picks).  kNested: the nested DDA instead
-// (a stage's choice, kDdaNested: scenes whose rays stay coherent).
-template <bool kPick, bool kNested>
+// different lights, so they take the unified walk (Walk, vr_device.h).
+// kNested: the nested DDA instead (a stage's choice, kDdaNested).
+template <bool kNested>
 __device__ __forceinline__ bool light_occluded(const WorldView& w, uint32_t lpos, uint32_t lsize, f3 spo, f3 L,
                                                int steps)
 {
     float dist = 0.0f;
     uint32_t side = 0;
     const uint32_t v = kNested ? trace<kTraceOpaque>(w, spo, L, steps, 0u, dist, side)
-                               : (kPick ? trace_sched(w, spo, L, steps, dist, side)
-                                        : trace_sched_walk<true>(w, spo, L, steps, dist, side));
+                               : trace_free<kTraceOpaque>(w, spo, L, steps, dist, side);
     if (v == 0u) return true;
     const f3 N = voxel_normal(side, L);
     const uint32_t hx = f2u((L.x * dist + spo.x) - N.x * 0.1f);
@@ -454,7 +448,7 @@ __device__ __forceinline__ void initial_px(const FrameArgs& a, int x, int y)
             const float4 lb = a.L.b[res.light];
             const float4 la = a.L.a[res.light];
             const f3 L = normalize(sub(res.pos, spo));
-            occ = light_occluded<true, kNested>(a.w, __float_as_uint(lb.w), (uint32_t)la.w, spo, L, a.shadowSteps);
+            occ = light_occluded<kNested>(a.w, __float_as_uint(lb.w), (uint32_t)la.w, spo, L, a.shadowSteps);
             shadow = kTraced | (occ ? 0u : kVisible);
             traced = 1u;
         }
@@ -707,7 +701,7 @@ __device__ __forceinline__ float mis_weight_tile(const FrameArgs& a, int x, int 
             const f3 spo = f3{sh.sp.x + 0.1f * sh.N.x, sh.sp.y + 0.1f * sh.N.y, sh.sp.z + 0.1f * sh.N.z};
             const f3 Ld = normalize(sub(f3{smp.x, smp.y, smp.z}, spo));
             const float4 tla = a.L.a[light], tlb = a.L.b[light];
-            if (light_occluded<true, kNested>(a.w, __float_as_uint(tlb.w), (uint32_t)tla.w, spo, Ld, a.shadowSteps))
+            if (light_occluded<kNested>(a.w, __float_as_uint(tlb.w), (uint32_t)tla.w, spo, Ld, a.shadowSteps))
                 atomicOr(&L.occluded[owner], 1u << (tk >> 8));
         }
         __syncthreads();
@@ -794,7 +788,7 @@ __device__ __forceinline__ bool shade_px(const FrameArgs& a, int x, int y)
                     if (kDefer && known < 0) return true;
                     const bool visible =
                         known >= 0 ? known == 1
-                                   : !light_occluded<false, kNested>(a.w, __float_as_uint(lb.w), (uint32_t)la.w, spo, L, a.shadowSteps);
+                                   : !light_occluded<kNested>(a.w, __float_as_uint(lb.w), (uint32_t)la.w, spo, L, a.shadowSteps);
                     // what the traversal did not keep in registers: from LDS
                     // when parked, else the values themselves
                     const float4 pp = park ? vload(pk.p[t]) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -861,15 +855,15 @@ __device__ __forceinline__ void stage_uber(const uint32_t* __restrict__ src)
     __syncthreads();
 }
 
-// kTraces: the stage traces rays (and so reads the staged uber grid)
-template <bool kTraces = true, class F>
+// kStage: the stage traces with the nested DDA (and so reads the staged uber grid)
+template <bool kStage, class F>
 __device__ __forceinline__ void one_view(const FrameArgs& a, F f)
 {
-    if (kTraces) stage_uber(a.w.uber);
+    if (kStage) stage_uber(a.w.uber);
     int x, y;
     tile_pixel(a.tileOrder, x, y);
     FrameArgs b = a;
-    if (kTraces) b.w.uber = uber_lds();
+    if (kStage) b.w.uber = uber_lds();
     if (x < (int)a.W && y < (int)a.H) f(b, x, y);
 }
 
@@ -883,18 +877,19 @@ __device__ __forceinline__ void one_view(const FrameArgs& a, F f)
 // the staging barriers.
 // kAll: f runs on every thread of the tile (it checks the bounds itself and
 // may use barriers); otherwise only on the pixels inside the view.
-template <bool kAll = false, class F>
+// kStage: f traces with the nested DDA.
+template <bool kAll, bool kStage, class F>
 __device__ __forceinline__ void view_tile(const ViewChunk& c, uint32_t t, uint32_t& staged, F f)
 {
     uint32_t v = 0;
     while (v + 1 < c.n && c.start[v + 1] <= t) v++;
-    if (v != staged) {
+    if (kStage && v != staged) {
         if (staged != ~0u) __syncthreads();  // the previous view's tile is done with LDS
         stage_uber(c.v[v].w.uber);
         staged = v;
     }
     FrameArgs a = c.v[v];
-    a.w.uber = uber_lds();
+    if (kStage) a.w.uber = uber_lds();
     const uint32_t lt = t - c.start[v];
     const uint32_t tilesX = (a.W + 15u) >> 4;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -904,16 +899,16 @@ __device__ __forceinline__ void view_tile(const ViewChunk& c, uint32_t t, uint32
 }
 
 // kPersistent: gridDim.x < total, each block loops; otherwise one tile per block
-template <bool kPersistent, bool kAll = false, class F>
+template <bool kPersistent, bool kAll, bool kStage, class F>
 __device__ __forceinline__ void many_views(const ViewChunk& c, F f)
 {
     const uint32_t total = c.start[c.n];
     uint32_t staged = ~0u;
     if (!kPersistent) {
-        if (blockIdx.x < total) view_tile<kAll>(c, blockIdx.x, staged, f);
+        if (blockIdx.x < total) view_tile<kAll, kStage>(c, blockIdx.x, staged, f);
         return;
     }
-    for (uint32_t t = blockIdx.x; t < total; t += gridDim.x) view_tile<kAll>(c, t, staged, f);
+    for (uint32_t t = blockIdx.x; t < total; t += gridDim.x) view_tile<kAll, kStage>(c, t, staged, f);
 }
 
 // Occupancy targets (waves per SIMD) of the ray-tracing stages: their DDA
@@ -929,12 +924,12 @@ __device__ __forceinline__ void many_views(const ViewChunk& c, F f)
 template <int W>
 __global__ __launch_bounds__(256) VR_WAVES(W) void k_primary(FrameArgs a)
 {
-    one_view(a, [](const FrameArgs& v, int x, int y) { primary_px(v, x, y); });
+    one_view<true>(a, [](const FrameArgs& v, int x, int y) { primary_px(v, x, y); });
 }
 template <int W, bool kNested>
 __global__ __launch_bounds__(256) VR_WAVES(W) void k_initial(FrameArgs a)
 {
-    one_view(a, [](const FrameArgs& v, int x, int y) { initial_px<kNested>(v, x, y); });
+    one_view<kNested>(a, [](const FrameArgs& v, int x, int y) { initial_px<kNested>(v, x, y); });
 }
 // Spatial reuse, then shading of the tile's 256 pixels.  Only the pixels
 // whose final sample needs a shadow ray the candidate pass did not trace
@@ -1001,11 +996,11 @@ __device__ __forceinline__ void resolve_tile(const FrameArgs& a, int x, int y)
 template <bool kMis, int W, bool kNested>
 __global__ __launch_bounds__(256) VR_WAVES(W) void k_resolve(FrameArgs a)
 {
-    stage_uber(a.w.uber);
+    if (kNested) stage_uber(a.w.uber);
     int x, y;
     tile_pixel(a.tileOrder, x, y);
     FrameArgs b = a;
-    b.w.uber = uber_lds();
+    if (kNested) b.w.uber = uber_lds();
     resolve_tile<kMis, kNested>(b, x, y);
 }
 
@@ -1129,9 +1124,9 @@ __global__ __launch_bounds__(256) VR_WAVES(8) void k_mis_trace(FrameArgs a, MisB
     // workgroups past the count leave at once (workgroup 0 counts the rays)
     const uint32_t n = *m.count;
     if (blockIdx.x * 256u >= n && blockIdx.x != 0u) return;
-    stage_uber(a.w.uber);
+    if (kNested) stage_uber(a.w.uber);
     FrameArgs b = a;
-    b.w.uber = uber_lds();
+    if (kNested) b.w.uber = uber_lds();
     if (blockIdx.x == 0u && threadIdx.x == 0u) count_rays(b.rays, kRaysMis, n);
     for (uint32_t t = blockIdx.x * 256u + threadIdx.x; t < n; t += gridDim.x * 256u) {
         const uint2 task = m.list[t];
@@ -1143,7 +1138,7 @@ __global__ __launch_bounds__(256) VR_WAVES(8) void k_mis_trace(FrameArgs a, MisB
         const f3 spo = f3{sh.sp.x + 0.1f * sh.N.x, sh.sp.y + 0.1f * sh.N.y, sh.sp.z + 0.1f * sh.N.z};
         const f3 Ld = normalize(sub(f3{__uint_as_float(smp.x), __uint_as_float(smp.y), __uint_as_float(smp.z)}, spo));
         const float4 tla = b.L.a[smp.w], tlb = b.L.b[smp.w];
-        if (light_occluded<true, kNested>(b.w, __float_as_uint(tlb.w), (uint32_t)tla.w, spo, Ld, b.shadowSteps))
+        if (light_occluded<kNested>(b.w, __float_as_uint(tlb.w), (uint32_t)tla.w, spo, Ld, b.shadowSteps))
             atomicOr(&m.occ[owner], 1u << k);
     }
 }
@@ -1151,11 +1146,11 @@ __global__ __launch_bounds__(256) VR_WAVES(8) void k_mis_trace(FrameArgs a, MisB
 template <int W, bool kNested>
 __global__ __launch_bounds__(256) VR_WAVES(W) void k_mis_finish(FrameArgs a, MisBufs m)
 {
-    stage_uber(a.w.uber);
+    if (kNested) stage_uber(a.w.uber);
     int x, y;
     tile_pixel(a.tileOrder, x, y);
     FrameArgs b = a;
-    b.w.uber = uber_lds();
+    if (kNested) b.w.uber = uber_lds();
     if (blockIdx.x == 0u && blockIdx.y == 0u && threadIdx.x == 0u) *m.count = 0u;  // the tracer has read it
     const bool in = x < (int)b.W && y < (int)b.H;
     if (in) {
@@ -1198,12 +1193,12 @@ __global__ __launch_bounds__(256) VR_WAVES(W) void k_mis_finish(FrameArgs a, Mis
 template <bool kPersistent>
 __global__ __launch_bounds__(256) VR_WAVES(8) void k_primary_views(ViewChunk c)
 {
-    many_views<kPersistent>(c, [](const FrameArgs& v, int x, int y) { primary_px(v, x, y); });
+    many_views<kPersistent, false, true>(c, [](const FrameArgs& v, int x, int y) { primary_px(v, x, y); });
 }
 template <bool kPersistent>
 __global__ __launch_bounds__(256) VR_WAVES(7) void k_initial_views(ViewChunk c)
 {
-    many_views<kPersistent>(c, [](const FrameArgs& v, int x, int y) { initial_px<false>(v, x, y); });
+    many_views<kPersistent, false, false>(c, [](const FrameArgs& v, int x, int y) { initial_px<false>(v, x, y); });
 }
 // kAnyMis: some view merges with MIS weights (the kernel then carries the
 // MIS variant's registers).  Batch frames do not overlap one another, so the
@@ -1211,7 +1206,7 @@ __global__ __launch_bounds__(256) VR_WAVES(7) void k_initial_views(ViewChunk c)
 template <bool kPersistent, bool kAnyMis>
 __global__ __launch_bounds__(256) VR_WAVES(kAnyMis ? kDefaultWavesMis : 7) void k_resolve_views(ViewChunk c)
 {
-    many_views<kPersistent, true>(c, [](const FrameArgs& v, int x, int y) {
+    many_views<kPersistent, true, false>(c, [](const FrameArgs& v, int x, int y) {
         if (kAnyMis && v.misSpatial) resolve_tile<true, false>(v, x, y);
         else resolve_tile<false, false, !kAnyMis>(v, x, y);
     });
@@ -1222,15 +1217,28 @@ __global__ __launch_bounds__(256) VR_WAVES(kAnyMis ? kDefaultWavesMis : 7) void 
 // ---------------------------------------------------------------------------
 
 // commit (cl/kernels.cl:448-477): one 128-thread group per staged brick,
-// 16 bytes per thread
+// 16 bytes per thread, and the brick's occupied slabs
 __global__ __launch_bounds__(128) void k_commit(const uint32_t* __restrict__ ids, const uint4* __restrict__ src,
-                                                uint4* __restrict__ pool, uint32_t n, uint32_t cap)
+                                                uint4* __restrict__ pool, uint32_t* __restrict__ proj, uint32_t n,
+                                                uint32_t cap)
 {
+    __shared__ uint32_t slabs;
     const uint32_t b = blockIdx.x;
     if (b >= n) return;
     const uint32_t id = ids[b];
     if (id >= cap) return;
-    pool[(size_t)id * 128u + threadIdx.x] = src[(size_t)b * 128u + threadIdx.x];
+    if (threadIdx.x == 0u) slabs = 0u;
+    __syncthreads();
+    const uint4 v = src[(size_t)b * 128u + threadIdx.x];
+    pool[(size_t)id * 128u + threadIdx.x] = v;
+    // voxels 4 i .. 4 i + 3 of thread i: x = 4 (i & 1) + 0..3
+    const uint32_t i = threadIdx.x, x = (i & 1u) * 4u, y = (i >> 1) & 7u, z = i >> 4;
+    uint32_t m = (v.x ? brick_slabs(x, y, z) : 0u) | (v.y ? brick_slabs(x + 1u, y, z) : 0u) |
+                 (v.z ? brick_slabs(x + 2u, y, z) : 0u) | (v.w ? brick_slabs(x + 3u, y, z) : 0u);
+    for (uint32_t o = 32u; o > 0u; o >>= 1) m |= (uint32_t)__shfl_xor((int)m, (int)o, 64);
+    if ((i & 63u) == 0u) atomicOr(&slabs, m);
+    __syncthreads();
+    if (i == 0u) proj[id] = slabs;
 }
 
 // updateUberGrid (cl/kernels.cl:498-513), stored as bits: cell
@@ -1252,6 +1260,20 @@ __global__ __launch_bounds__(256) void k_uber(const uint32_t* __restrict__ grid,
     if (lane == 32u) uber[task >> 5] = (uint32_t)(bits >> 32);
 }
 
+// The top and uber cells as the unified walk reads them (vr_device.h): a wave
+// per uber cell, a lane per top cell of its block, so the block is written
+// in one 256-byte run.
+__global__ __launch_bounds__(256) void k_walk_cells(const uint32_t* __restrict__ grid, uint32_t* __restrict__ cells)
+{
+    const uint32_t u = blockIdx.x * 4u + (threadIdx.x >> 6), l = threadIdx.x & 63u;  // 32768 uber cells: the grid is exact
+    const uint32_t ux = u & 31u, uy = (u >> 5) & 31u, uz = u >> 10;
+    const uint32_t x = ux * 4u + (l & 3u), y = uy * 4u + ((l >> 2) & 3u), z = uz * 4u + (l >> 4);
+    const uint32_t c = grid[x + z * 128u + y * 16384u];
+    cells[(size_t)u * 64u + l] = (c & 1u) ? kChild | (c >> 1) : c >> 1;
+    const uint64_t any = __ballot(c != 0u);
+    if (l == 0u) cells[kTopWords + u] = any != 0u ? kChild : 0u;
+}
+
 // traceBatch (cl/kernels.cl:395-417) returning voxel, dist, side
 __global__ __launch_bounds__(256) void k_trace_batch(WorldView w, const float* __restrict__ O, const float* __restrict__ D,
                                                      uint32_t n, uint32_t kind, int32_t steps, uint32_t* voxel,
@@ -1263,7 +1285,7 @@ __global__ __launch_bounds__(256) void k_trace_batch(WorldView w, const float* _
     const f3 B = f3{D[3 * i], D[3 * i + 1], D[3 * i + 2]};
     float d = 0.0f;
     uint32_t s = 0;
-    const uint32_t v = kind == 1u ? trace_sched(w, A, B, steps, d, s) : trace<kTraceAll>(w, A, B, steps, 0u, d, s);
+    const uint32_t v = kind == 1u ? trace_free<kTraceOpaque>(w, A, B, steps, d, s) : trace_free<kTraceAll>(w, A, B, steps, d, s);
     voxel[i] = v;
     dist[i] = v ? d : 0.0f;
     side[i] = v ? s : 0u;
@@ -1466,18 +1488,19 @@ hipError_t stage_views_node(int stage, const ViewChunk* c, uint32_t blocks, bool
     return hipSuccess;
 }
 
-hipError_t launch_commit(const uint32_t* ids, const uint32_t* src, uint32_t* pool, uint32_t n, uint32_t cap,
-                         hipStream_t s)
+hipError_t launch_commit(const uint32_t* ids, const uint32_t* src, uint32_t* pool, uint32_t* proj, uint32_t n,
+                         uint32_t cap, hipStream_t s)
 {
     if (n == 0) return hipSuccess;
     hipLaunchKernelGGL(k_commit, dim3(n), dim3(128), 0, s, ids, reinterpret_cast<const uint4*>(src),
-                       reinterpret_cast<uint4*>(pool), n, cap);
+                       reinterpret_cast<uint4*>(pool), proj, n, cap);
     return hipGetLastError();
 }
 
-hipError_t launch_uber(const uint32_t* grid, uint32_t* uber, hipStream_t s)
+hipError_t launch_uber(const uint32_t* grid, uint32_t* uber, uint32_t* cells, hipStream_t s)
 {
     hipLaunchKernelGGL(k_uber, dim3(128), dim3(256), 0, s, grid, uber);
+    hipLaunchKernelGGL(k_walk_cells, dim3(kUberWords / 4u), dim3(256), 0, s, grid, cells);
     return hipGetLastError();
 }
 

@@ -96,7 +96,8 @@ struct vr_ctx {
     // world
     uint32_t* grid = nullptr;       // [128^3]
     uint32_t* uber = nullptr;       // [32^3 bits]
-    uint32_t* bricks = nullptr;     // [brick_capacity * 512]
+    uint32_t* bricks = nullptr;     // [brick_capacity * 512], then the unified walk's cells
+    uint32_t* proj = nullptr;       // [brick_capacity] WorldView::proj
     uint32_t* stageIds = nullptr;   // [VR_MAXCOMMITS]
     uint32_t* stageData = nullptr;  // [VR_MAXCOMMITS * 512]
     // lights
@@ -335,11 +336,19 @@ bool finite_camera(const vr_render_params* p)
     return true;
 }
 
+// word index of the unified walk's cells, behind the pool's voxels
+size_t cells_at(const vr_ctx* c) { return (size_t)c->cfg.brick_capacity * VR_BRICKSIZE; }
+
+WorldView world_view(const vr_ctx* c)
+{
+    return WorldView{c->grid, c->bricks, c->uber, c->proj, (uint32_t)cells_at(c)};
+}
+
 FrameArgs frame_args(const vr_ctx* c, const vr_render_params* p)
 {
     FrameArgs a;
     std::memset(&a, 0, sizeof(a));
-    a.w = WorldView{c->grid, c->bricks, c->uber};
+    a.w = world_view(c);
     a.L = LightView{c->la, c->lb, c->pick, p ? p->numberOfLights : 0u};
     if (p) {
         a.cam.ox = p->oneOverRes[0], a.cam.oy = p->oneOverRes[1];
@@ -516,7 +525,7 @@ int vr_create(const vr_config* cfg, vr_ctx** out)
     for (int f = 0; good && f < kRing; f++)
         for (int i = 0; good && i < 2 * VR_NUM_STAGES; i++) good = ok(hipEventCreate(&c->ev[f][i]));
     good = good && ok(dalloc(&c->grid, VR_GRIDSIZE)) && ok(dalloc(&c->uber, 1024)) &&
-           ok(dalloc(&c->bricks, (size_t)cfg->brick_capacity * VR_BRICKSIZE)) &&
+           ok(dalloc(&c->bricks, cells_at(c) + kTopWords + kUberWords)) && ok(dalloc(&c->proj, cfg->brick_capacity)) &&
            ok(dalloc(&c->stageIds, VR_MAXCOMMITS)) && ok(dalloc(&c->stageData, (size_t)VR_MAXCOMMITS * VR_BRICKSIZE)) &&
            ok(dalloc(&c->emitLut, 256)) && ok(dalloc(&c->frame, n)) && ok(dalloc(&c->rays, (size_t)kRayKinds));
     for (int i = 0; good && i < 2; i++)
@@ -525,7 +534,8 @@ int vr_create(const vr_config* cfg, vr_ctx** out)
     if (good) {
         good = ok(hipMemsetAsync(c->grid, 0, (size_t)VR_GRIDSIZE * 4, c->stream)) &&
                ok(hipMemsetAsync(c->uber, 0, 4096, c->stream)) &&
-               ok(hipMemsetAsync(c->bricks, 0, (size_t)cfg->brick_capacity * VR_BRICKSIZE * 4, c->stream)) &&
+               ok(hipMemsetAsync(c->bricks, 0, (cells_at(c) + kTopWords + kUberWords) * 4, c->stream)) &&
+               ok(hipMemsetAsync(c->proj, 0, (size_t)cfg->brick_capacity * 4, c->stream)) &&
                ok(hipMemcpyAsync(c->emitLut, cfg->emit_lut, 256 * 4, hipMemcpyHostToDevice, c->stream)) &&
                ok(hipMemsetAsync(c->frame, 0, n * 16, c->stream));
         for (int i = 0; good && i < 2; i++)
@@ -554,7 +564,7 @@ int vr_destroy(vr_ctx* c)
     if (c->counted) g_liveContexts--;
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     if (c->side) (void)hipStreamSynchronize(c->side);
-    dfree(c->grid), dfree(c->uber), dfree(c->bricks), dfree(c->stageIds), dfree(c->stageData);
+    dfree(c->grid), dfree(c->uber), dfree(c->bricks), dfree(c->proj), dfree(c->stageIds), dfree(c->stageData);
     dfree(c->la), dfree(c->lb), dfree(c->pick), dfree(c->emitLut), dfree(c->frame);
     dfree(c->rays);
     for (int i = 0; i < 2; i++) {
@@ -604,10 +614,10 @@ int vr_commit(vr_ctx* c, const uint32_t* grid, const uint32_t* ids, const uint32
         HIPCHK(c, hipMemcpyAsync(c->stageIds, ids + done, (size_t)k * 4, hipMemcpyHostToDevice, c->stream));
         HIPCHK(c, hipMemcpyAsync(c->stageData, payload + (size_t)done * VR_BRICKSIZE, (size_t)k * VR_BRICKSIZE * 4,
                                  hipMemcpyHostToDevice, c->stream));
-        HIPCHK(c, launch_commit(c->stageIds, c->stageData, c->bricks, k, cap, c->stream));
+        HIPCHK(c, launch_commit(c->stageIds, c->stageData, c->bricks, c->proj, k, cap, c->stream));
         done += k;
     }
-    HIPCHK(c, launch_uber(c->grid, c->uber, c->stream));
+    HIPCHK(c, launch_uber(c->grid, c->uber, c->bricks + cells_at(c), c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     c->committed = true;
     return VR_OK;
@@ -965,7 +975,7 @@ int vr_trace_rays(vr_ctx* c, const float* O, const float* D, uint32_t n, uint32_
         hipError_t e = hipMemcpyAsync(dO, O, (size_t)n * 12, hipMemcpyHostToDevice, c->stream);
         if (e == hipSuccess) e = hipMemcpyAsync(dD, D, (size_t)n * 12, hipMemcpyHostToDevice, c->stream);
         if (e == hipSuccess)
-            e = launch_trace_batch(WorldView{c->grid, c->bricks, c->uber}, dO, dD, n, kind, steps, dv, dd, ds, c->stream);
+            e = launch_trace_batch(world_view(c), dO, dD, n, kind, steps, dv, dd, ds, c->stream);
         if (e == hipSuccess) e = hipMemcpyAsync(voxel, dv, (size_t)n * 4, hipMemcpyDeviceToHost, c->stream);
         if (e == hipSuccess) e = hipMemcpyAsync(dist, dd, (size_t)n * 4, hipMemcpyDeviceToHost, c->stream);
         if (e == hipSuccess) e = hipMemcpyAsync(side, ds, (size_t)n * 4, hipMemcpyDeviceToHost, c->stream);
@@ -1007,7 +1017,7 @@ int vr_trace_rays_noalloc(vr_ctx* c, const float* O, const float* D, uint32_t n,
     hipError_t e = hipMemcpyAsync(dO, O, (size_t)n * 12, hipMemcpyHostToDevice, c->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(dD, D, (size_t)n * 12, hipMemcpyHostToDevice, c->stream);
     if (e == hipSuccess)
-        e = launch_trace_batch(WorldView{c->grid, c->bricks, c->uber}, dO, dD, n, kind, steps, dv, dd, ds, c->stream);
+        e = launch_trace_batch(world_view(c), dO, dD, n, kind, steps, dv, dd, ds, c->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(voxel, dv, (size_t)n * 4, hipMemcpyDeviceToHost, c->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(dist, dd, (size_t)n * 4, hipMemcpyDeviceToHost, c->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(side, ds, (size_t)n * 4, hipMemcpyDeviceToHost, c->stream);
@@ -1370,11 +1380,11 @@ int vr_scene_step(vr_ctx* c, uint32_t frame, uint32_t seed, uint32_t edit_permil
                                    "brick capacity");
     HIPCHK(c, hipSetDevice(c->device));
     c->worldEpoch++;  // the next primary pass waits for these edits
-    HIPCHK(c, launch_edit_bricks(c->bricks, high_water, frame, seed, edit_permille, walk_steps, c->stream));
+    HIPCHK(c, launch_edit_bricks(c->bricks, c->proj, high_water, frame, seed, edit_permille, walk_steps, c->stream));
     if (c->motionN > 0 && c->motionN == c->nLights) {
         const LightMotionView m{c->la, c->lb, c->lightPos, c->lightVel, c->lightVoxel, c->lightTarget, c->claim,
                                 c->motionN};
-        HIPCHK(c, launch_move_lights(m, c->grid, c->bricks, c->cfg.brick_capacity, c->stream));
+        HIPCHK(c, launch_move_lights(m, c->grid, c->bricks, c->proj, c->cfg.brick_capacity, c->stream));
     }
     return VR_OK;
 }
