@@ -146,8 +146,8 @@ struct MisBufs {
     uint4* info;      // [W*H] taps whose ray is listed, combined taps, sel + 1, own M
     float2* terms;    // [tap][W*H] M * T and T of each combined tap
 };
-// traceBlocks: workgroups of the tracer's grid (256 rays each), enough for
-// the list's capacity
+// traceBlocks: workgroups of the tracer's grid at 256 rays each, enough for
+// the list's capacity (the refilling walk takes no more than fit the chip)
 hipError_t launch_mis_split(const FrameArgs& a, const MisBufs& m, uint32_t traceBlocks, hipStream_t s);
 // Up to kChunkViews views rendered by one launch per stage: their
 // FrameArgs travel in the kernel argument (8 x 472 B + the tile table,

@@ -86,7 +86,18 @@ __device__ __forceinline__ void count_rays(unsigned long long* rays, int k, uint
     if (rays && n) atomicAdd(&rays[k], (unsigned long long)n);
 }
 
-// GridCoordinatesFromHit + Uint3CubeEquals (cl/tools.cl:452-472) behind
+// GridCoordinatesFromHit + Uint3CubeEquals (cl/tools.cl:452-472): the hit of
+// a shadow ray from spo along L lies inside the light's cube
+__device__ __forceinline__ bool hit_inside_light(uint32_t side, float dist, uint32_t lpos, uint32_t lsize, f3 spo, f3 L)
+{
+    const f3 N = voxel_normal(side, L);
+    const uint32_t hx = f2u((L.x * dist + spo.x) - N.x * 0.1f);
+    const uint32_t hy = f2u((L.y * dist + spo.y) - N.y * 0.1f);
+    const uint32_t hz = f2u((L.z * dist + spo.z) - N.z * 0.1f);
+    const uint32_t ly = lpos >> 20, lz = (lpos >> 10) & 1023u, lx = lpos & 1023u;
+    return lx <= hx && lx + lsize > hx && ly <= hy && ly + lsize > hy && lz <= hz && lz + lsize > hz;
+}
+
 // isLightOccluded (cl/ris.cl:1-17).  A shadow ray that finds no opaque voxel
 // within its step budget counts as occluded.  Shadow rays of a wave head to
 // different lights, so they take the unified walk (Walk, vr_device.h).
@@ -99,14 +110,7 @@ __device__ __forceinline__ bool light_occluded(const WorldView& w, uint32_t lpos
     uint32_t side = 0;
     const uint32_t v = kNested ? trace<kTraceOpaque>(w, spo, L, steps, 0u, dist, side)
                                : trace_free<kTraceOpaque>(w, spo, L, steps, dist, side);
-    if (v == 0u) return true;
-    const f3 N = voxel_normal(side, L);
-    const uint32_t hx = f2u((L.x * dist + spo.x) - N.x * 0.1f);
-    const uint32_t hy = f2u((L.y * dist + spo.y) - N.y * 0.1f);
-    const uint32_t hz = f2u((L.z * dist + spo.z) - N.z * 0.1f);
-    const uint32_t ly = lpos >> 20, lz = (lpos >> 10) & 1023u, lx = lpos & 1023u;
-    const bool inside = lx <= hx && lx + lsize > hx && ly <= hy && ly + lsize > hy && lz <= hz && lz + lsize > hz;
-    return !inside;
+    return v == 0u || !hit_inside_light(side, dist, lpos, lsize, spo, L);
 }
 
 // same-face test of temporal / spatial reuse; hit words carry side (bits
@@ -1117,30 +1121,76 @@ __global__ __launch_bounds__(256) VR_WAVES(W) void k_mis_list(FrameArgs a, MisBu
     }
 }
 
+// Ray `task` of the list: from the neighbour's shading point to the merged
+// sample of the owner (stored by k_mis_list)
+struct MisRay {
+    f3 spo, L;
+    uint32_t light;
+};
+
+__device__ __forceinline__ MisRay mis_ray(const FrameArgs& a, uint2 task)
+{
+    const uint32_t owner = task.x >> 5, ni = task.y;
+    const uint4 smp = a.A.r1[owner];
+    const int nx = (int)(ni % a.W), ny = (int)(ni / a.W);
+    const float nd = __uint_as_float(a.B.r0[ni].y);
+    const Shading sh = shading_at(a, nx, ny, a.cur.hitw[ni], nd);
+    MisRay r;
+    r.spo = f3{sh.sp.x + 0.1f * sh.N.x, sh.sp.y + 0.1f * sh.N.y, sh.sp.z + 0.1f * sh.N.z};
+    r.L = normalize(sub(f3{__uint_as_float(smp.x), __uint_as_float(smp.y), __uint_as_float(smp.z)}, r.spo));
+    r.light = smp.w;
+    return r;
+}
+
+// what a lane's ray needs again when it has ended
+struct RayLds {
+    float4 o[256], d[256];  // origin and light, direction and where its answer goes
+};
+
+__device__ __forceinline__ RayLds& ray_lds()
+{
+    __shared__ RayLds l;
+    return l;
+}
+
 template <bool kNested>
 __global__ __launch_bounds__(256) VR_WAVES(8) void k_mis_trace(FrameArgs a, MisBufs m)
 {
-    // one thread per listed ray: the grid covers the list's capacity and the
-    // workgroups past the count leave at once (workgroup 0 counts the rays)
     const uint32_t n = *m.count;
     if (blockIdx.x * 256u >= n && blockIdx.x != 0u) return;
-    if (kNested) stage_uber(a.w.uber);
-    FrameArgs b = a;
-    if (kNested) b.w.uber = uber_lds();
-    if (blockIdx.x == 0u && threadIdx.x == 0u) count_rays(b.rays, kRaysMis, n);
-    for (uint32_t t = blockIdx.x * 256u + threadIdx.x; t < n; t += gridDim.x * 256u) {
-        const uint2 task = m.list[t];
-        const uint32_t owner = task.x >> 5, k = task.x & 31u, ni = task.y;
-        const uint4 smp = b.A.r1[owner];  // the merged sample, stored by k_mis_list
-        const int nx = (int)(ni % b.W), ny = (int)(ni / b.W);
-        const float nd = __uint_as_float(b.B.r0[ni].y);
-        const Shading sh = shading_at(b, nx, ny, b.cur.hitw[ni], nd);
-        const f3 spo = f3{sh.sp.x + 0.1f * sh.N.x, sh.sp.y + 0.1f * sh.N.y, sh.sp.z + 0.1f * sh.N.z};
-        const f3 Ld = normalize(sub(f3{__uint_as_float(smp.x), __uint_as_float(smp.y), __uint_as_float(smp.z)}, spo));
-        const float4 tla = b.L.a[smp.w], tlb = b.L.b[smp.w];
-        if (light_occluded<kNested>(b.w, __float_as_uint(tlb.w), (uint32_t)tla.w, spo, Ld, b.shadowSteps))
-            atomicOr(&m.occ[owner], 1u << k);
+    if (blockIdx.x == 0u && threadIdx.x == 0u) count_rays(a.rays, kRaysMis, n);
+    if (kNested) {
+        stage_uber(a.w.uber);
+        WorldView w = a.w;
+        w.uber = uber_lds();
+        for (uint32_t t = blockIdx.x * 256u + threadIdx.x; t < n; t += gridDim.x * 256u) {
+            const uint2 task = m.list[t];
+            const MisRay r = mis_ray(a, task);
+            const float4 tla = a.L.a[r.light], tlb = a.L.b[r.light];
+            if (light_occluded<true>(w, __float_as_uint(tlb.w), (uint32_t)tla.w, r.spo, r.L, a.shadowSteps))
+                atomicOr(&m.occ[task.x >> 5], 1u << (task.x & 31u));
+        }
+        return;
     }
+    RayLds& l = ray_lds();
+    const uint32_t t = threadIdx.x;
+    walk_list<kTraceOpaque>(
+        a.w, a.shadowSteps, n,
+        [&](uint32_t i, f3& A, f3& B) {
+            const uint2 task = m.list[i];
+            const MisRay r = mis_ray(a, task);
+            l.o[t] = make_float4(r.spo.x, r.spo.y, r.spo.z, __uint_as_float(r.light));
+            l.d[t] = make_float4(r.L.x, r.L.y, r.L.z, __uint_as_float(task.x));
+            A = r.spo, B = r.L;
+        },
+        [&](const Walk<kTraceOpaque>& k) {
+            const float4 o = vload(l.o[t]), d = vload(l.d[t]);
+            const uint32_t light = __float_as_uint(o.w), task = __float_as_uint(d.w);
+            const float4 tla = a.L.a[light], tlb = a.L.b[light];
+            if (k.mode == kMiss || !hit_inside_light(k.last, k.distance(), __float_as_uint(tlb.w), (uint32_t)tla.w,
+                                                     f3{o.x, o.y, o.z}, f3{d.x, d.y, d.z}))
+                atomicOr(&m.occ[task >> 5], 1u << (task & 31u));
+        });
 }
 
 template <int W, bool kNested>
@@ -1419,6 +1469,11 @@ static const void* mis_kernel(int which, uint32_t waves, bool nested)
     }
 }
 
+// Workgroups of a refilling trace's grid: 256 CUs x the 8 that fit each.
+// Fewer waves take more rays each but hide less latency (moving 1920x1080
+// scene, whole frames: 1024 workgroups 3.45 ms, 1280 3.37, 2048 3.28, 4096 3.31).
+static constexpr uint32_t kTraceBlocks = 2048u;
+
 hipError_t launch_mis_split(const FrameArgs& a, const MisBufs& m, uint32_t traceBlocks, hipStream_t s)
 {
     if (a.dda > kDdaNested || traceBlocks == 0u) return hipErrorInvalidValue;
@@ -1426,6 +1481,9 @@ hipError_t launch_mis_split(const FrameArgs& a, const MisBufs& m, uint32_t trace
     const void* k0 = mis_kernel(0, a.waves, nested);
     const void* k2 = mis_kernel(1, a.waves, nested);
     if (!k0 || !k2) return hipErrorInvalidValue;
+    // nested: a thread per ray of the list's capacity; the refilling walk:
+    // at most the waves that fit the chip
+    if (!nested) traceBlocks = traceBlocks < kTraceBlocks ? traceBlocks : kTraceBlocks;
     const void* k1 = nested ? reinterpret_cast<const void*>(&k_mis_trace<true>)
                             : reinterpret_cast<const void*>(&k_mis_trace<false>);
     void* args[] = {const_cast<FrameArgs*>(&a), const_cast<MisBufs*>(&m)};
