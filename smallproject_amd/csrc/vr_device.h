@@ -348,12 +348,15 @@ __device__ uint32_t trace(const WorldView& w, f3 A, f3 B, int steps, uint32_t th
 // chosen by how many lanes wait for each (ballot counts, a scalar branch).
 // Every lane performs trace()'s operations in its order, so hits, distances
 // and sides are the same bits; what differs is which lanes run together.
-// The waves' issue slots are what bounds it.  Against the walk that ran one
-// of the three levels per turn (a wave of 64 shadow rays on c2's frames:
-// 288 turns, 8-14 lanes busy in each; here 141), whole frames at 1920x1080:
-// 2.48 -> 1.99 ms (c2, uniform lights), 2.29 -> 1.71 ms (letters at
-// 1600x1024, where trace() had been the faster of the two), 3.48 -> 2.40 ms
-// (many-light world at 1279x717, MIS merge).
+// The waves' issue slots are what bounds it, so a step turn is kept to about
+// 31 vector instructions and a change turn to about 105: what a lane does
+// next is held in lane masks (scalar registers, whose instructions issue
+// beside the vector ones), a lane's cell in bytes whose dot product with the
+// level's weights is its word.  Against the walk that ran one of the three
+// levels per turn (a wave of 64 shadow rays on c2's frames: 288 turns, 8-14
+// lanes busy in each; here 141), whole frames: c2 at 1920x1080 2.48 -> 1.81
+// ms, letters at 1600x1024 2.29 -> 1.62 ms (trace() had been the faster of
+// the two there).
 //
 // Brick walks that cannot hit are left out.  A walk that leaves its brick
 // without a hit changes nothing but `t` and `last`, which the parent's step
@@ -368,15 +371,24 @@ __device__ uint32_t trace(const WorldView& w, f3 A, f3 B, int steps, uint32_t th
 // brick walks are left out, 14 of its 25 voxel steps.
 constexpr float kSlack = 0.0625f;
 
-__device__ __forceinline__ uint32_t lanes(uint64_t mask) { return (uint32_t)__builtin_popcountll(mask); }
+// lanes in a mask, counted by a scalar instruction (the compiler compares
+// two popcounts with vector ones)
+__device__ __forceinline__ int lanes(uint64_t mask)
+{
+    int n;
+    asm("s_bcnt1_i32_b64 %0, %1" : "=s"(n) : "s"(mask) : "scc");
+    return n;
+}
+__device__ __forceinline__ uint64_t lanes_where(bool b) { return __builtin_amdgcn_ballot_w64(b); }
+__device__ __forceinline__ bool lane_in(uint64_t mask) { return __builtin_amdgcn_inverse_ballot_w64(mask); }
 
 // Parent levels' state of the workgroup's lanes (256 threads at most): the
 // uber cell's and the top cell's crossing distances and packed cell, and the
-// top block's first word.  In LDS, so that the walk fits the registers of
-// the kernels that trace.
+// top block's first word and cell.  In LDS, so that the walk fits the
+// registers of the kernels that trace.
 struct WalkLds {
     float tx[2][256], ty[2][256], tz[2][256];
-    uint32_t p[2][256], base[256];
+    uint32_t p[2][256], base[256], org[256];
 };
 
 __device__ __forceinline__ WalkLds& walk_lds()
@@ -385,54 +397,58 @@ __device__ __forceinline__ WalkLds& walk_lds()
     return l;
 }
 
-// what a lane does next: visit and step, nothing (its ray ended, or it has
-// none), or change its level
-enum WalkMode : uint32_t { kStep = 0u, kMiss = 1u, kHit = 2u, kIdle = 3u, kDown = 4u, kUp = 5u };
-
 template <int KIND>
 struct Walk {
+    // What each lane does next, as lane masks (uniform values: scalar
+    // registers and instructions, beside the vector ones that bound the
+    // walk): visit and step, go into a child block, go back to the parent;
+    // its ray has ended with a hit or without one.  `solid`: lanes whose
+    // rays walk every brick.
+    uint64_t step_, down_, up_, hit_, miss_, solid_;
     // the ray: origin (inside the map, or moved to its border), direction,
-    // 1/direction, packed cell steps; distance to the moved origin
+    // 1/direction, distance to the moved origin
     f3 A, V, rV;
-    uint32_t dx, dy, dz;
     float to;
-    uint32_t solid;  // ~0: walk every brick
-    // the level the lane is at: crossing distances, packed cell inside the
-    // block, the block's first word and first cell, bits per axis, the bits
-    // that a cell outside the block has, the budget of a visit
+    // the level the lane is at: crossing distances; the cell inside its block
+    // and the steps along the axes, packed in bytes x | y << 8 | z << 16; the
+    // bits that a cell outside the block has; each byte's weight in the
+    // cell's word; the block's first word and first cell (x << 20 | y << 10
+    // | z in the map's cells of that level); a visit's budget (4, 1 and 0
+    // from the uber level down).  An uber cell's z byte is 8 z, so that its
+    // weight 1024 fits a byte.
     float tx, ty, tz;
-    uint32_t p, base, org, s, outside;
+    uint32_t p, dx, dy, dz, outside, weights, base, org;
     int cost;
     float t;
-    uint32_t last, o, mode;  // o: the current cell or voxel
+    uint32_t last, o;  // o: the current cell or voxel
     int steps;
 
-    static constexpr uint32_t kOut5 = ~((31u << 20) | (31u << 10) | 31u);
-    static constexpr uint32_t kOut2 = ~((3u << 20) | (3u << 10) | 3u);
-    static constexpr uint32_t kOut3 = ~((7u << 20) | (7u << 10) | 7u);
+    static constexpr uint32_t kOut5 = 0xff00e0e0u, kOut2 = 0xfffcfcfcu, kOut3 = 0xfff8f8f8u;
+    static constexpr uint32_t kWeights5 = 1u | (32u << 8) | (128u << 16), kWeights2 = 1u | (4u << 8) | (16u << 16),
+                              kWeights3 = 1u | (8u << 8) | (64u << 16);
 
-    // word of packed cell c of a block with b bits per axis
-    static __device__ __forceinline__ uint32_t cell(uint32_t c, uint32_t b)
-    {
-        return ((((c & 1023u) << b) + __builtin_amdgcn_ubfe(c, 10u, 10u)) << b) + (c >> 20);
-    }
+    __device__ __forceinline__ uint32_t word() const { return __builtin_amdgcn_udot4(p, weights, base, false); }
 
-    // the ray's first cell; trace()'s set-up
-    __device__ __forceinline__ void begin(const WorldView& w, f3 A0, f3 B, int budget)
+    __device__ __forceinline__ void clear() { step_ = down_ = up_ = hit_ = miss_ = solid_ = 0u; }
+
+    // trace()'s set-up: the ray's first cell.  False when the ray misses the
+    // map; `free_`: the ray's bricks may be left out.  The caller enters the
+    // lane in the masks.
+    __device__ __forceinline__ bool begin(const WorldView& w, f3 A0, f3 B, int budget, bool& free_)
     {
         constexpr float kBound = 1048576.0f;
-        const bool bounded = fabsf(A0.x) <= kBound && fabsf(A0.y) <= kBound && fabsf(A0.z) <= kBound &&
-                             fabsf(B.x) <= kBound && fabsf(B.y) <= kBound && fabsf(B.z) <= kBound;
-        solid = bounded ? 0u : ~0u;
+        free_ = fabsf(A0.x) <= kBound && fabsf(A0.y) <= kBound && fabsf(A0.z) <= kBound && fabsf(B.x) <= kBound &&
+                fabsf(B.y) <= kBound && fabsf(B.z) <= kBound;
         if (fabsf(B.x) < 1e-8f) B.x = B.x < 0 ? -1e-8f : 1e-8f;
         if (fabsf(B.y) < 1e-8f) B.y = B.y < 0 ? -1e-8f : 1e-8f;
         if (fabsf(B.z) < 1e-8f) B.z = B.z < 0 ? -1e-8f : 1e-8f;
         A = A0, V = B;
         rV = f3{1.0f / V.x, 1.0f / V.y, 1.0f / V.z};
-        dx = V.x > 0 ? (1u << 20) : (0xfffu << 20);
-        dy = V.y > 0 ? (1u << 10) : 0xfffffc00u;
-        dz = V.z > 0 ? 1u : 0xffffffffu;
-        to = 0.0f, t = 0.0f, last = 0u, steps = budget, mode = kStep;
+        dx = V.x > 0 ? 1u : ~0u;
+        dy = V.y > 0 ? 1u << 8 : ~0u << 8;
+        dz = V.z > 0 ? 8u << 16 : ~7u << 16;
+        to = 0.0f, t = 0.0f, last = 0u, steps = budget;
+        bool inside = true;
         if (A.x < 0 || A.y < 0 || A.z < 0 || A.x > 1024.0f || A.y > 1024.0f || A.z > 1024.0f) {
             const float tx1 = -A.x * rV.x, tx2 = (1024.0f - A.x) * rV.x;
             float tmin = fminf(tx1, tx2), tmax = fmaxf(tx1, tx2);
@@ -440,127 +456,27 @@ struct Walk {
             tmin = fmaxf(tmin, fminf(ty1, ty2)), tmax = fminf(tmax, fmaxf(ty1, ty2));
             const float tz1 = -A.z * rV.z, tz2 = (1024.0f - A.z) * rV.z;
             tmin = fmaxf(tmin, fminf(tz1, tz2)), tmax = fminf(tmax, fmaxf(tz1, tz2));
-            if (tmax < tmin || tmax <= 0) mode = kMiss;
+            inside = !(tmax < tmin || tmax <= 0);
             A.x += tmin * V.x, A.y += tmin * V.y, A.z += tmin * V.z;
             to = tmin;
             if (A.y < 0.01f || A.y > (1024.0f - 1.01f)) last = 1;
             if (A.z < 0.01f || A.z > (1024.0f - 1.01f)) last = 2;
         }
         const uint32_t cx = min(f2u(A.x) >> 5, 31u), cy = min(f2u(A.y) >> 5, 31u), cz = min(f2u(A.z) >> 5, 31u);
-        p = (cx << 20) | (cy << 10) | cz;
+        p = cx | (cy << 8) | (cz << 19);
         tx = ((float)(cx + (V.x > 0 ? 1u : 0u)) - A.x * 0.03125f) * rV.x;
         ty = ((float)(cy + (V.y > 0 ? 1u : 0u)) - A.y * 0.03125f) * rV.y;
         tz = ((float)(cz + (V.z > 0 ? 1u : 0u)) - A.z * 0.03125f) * rV.z;
-        base = w.top + kTopWords, org = 0u, s = 5u, outside = kOut5, cost = 4;
-        o = w.bricks[(size_t)(base + cell(p, 5u))];
+        base = w.top + kTopWords, org = 0u, outside = kOut5, weights = kWeights5, cost = 4;
+        o = w.bricks[(size_t)word()];
+        return inside;
     }
 
-    // Lanes in kStep: visit the cell, then step to the next one; the others
-    // keep their state (selects instead of branches: the compiler copies
-    // registers across divergent joins).
-    __device__ __forceinline__ void step(const WorldView& w)
-    {
-        const bool mine = mode == kStep;
-        steps -= mine ? cost : 0;
-        const bool child = (int32_t)o < 0 && s != 3u;
-        const bool stops = KIND == kTraceAll ? o != 0u : (o & 0xf000u) == 0xf000u;
-        const bool go = mine && steps > 0 && !child && !stops;
-        const float tn = fminf(tx, fminf(ty, tz));
-        const bool sx = go && tn == tx, sy = go && tn == ty, sz = go && tn == tz;
-        tx += sx ? fabsf(rV.x) : 0.0f;
-        ty += sy ? fabsf(rV.y) : 0.0f;
-        tz += sz ? fabsf(rV.z) : 0.0f;
-        p += (sx ? dx : 0u) + (sy ? dy : 0u) + (sz ? dz : 0u);
-        last = go ? (sz ? 2u : (sy ? 1u : 0u)) : last;
-        t = go ? tn : t;
-        const bool out = go && (p & outside) != 0u;
-        uint32_t next = child ? kDown : (stops ? kHit : kStep);
-        next = steps <= 0 || out ? (s == 5u ? kMiss : kUp) : next;
-        mode = mine ? next : mode;
-        if (go && !out) {
-            uint32_t at = base + cell(p, s);
-            asm volatile("; step" : "+v"(at));  // keeps the load in this unit
-            o = w.bricks[(size_t)at];
-        }
-    }
+    __device__ __forceinline__ bool more_steps() const { return lanes(step_) > lanes(down_ | up_); }
 
-    // Lanes in kUp: back to the parent, whose pending step follows without
-    // another visit (an empty cell, its budget given back)
-    __device__ __forceinline__ void up_level(const WorldView& w)
-    {
-        WalkLds& l = walk_lds();
-        const bool brick = s == 3u;
-        const int k = brick ? 1 : 0;
-        tx = l.tx[k][threadIdx.x], ty = l.ty[k][threadIdx.x], tz = l.tz[k][threadIdx.x], p = l.p[k][threadIdx.x];
-        base = brick ? l.base[threadIdx.x] : w.top + kTopWords;
-        org = (org >> s) - p;  // a block's first cell is its parent's cell << s
-        s = brick ? 2u : 5u, outside = brick ? kOut2 : kOut5, cost = brick ? 1 : 4;
-        steps += cost, o = 0u, mode = kStep;
-    }
-
-    // one axis of the box test: the brick's slabs between local cells a and b
-    static __device__ __forceinline__ uint32_t slabs_between(uint32_t slabs, uint32_t a, uint32_t b)
-    {
-        const uint32_t n = (a > b ? a - b : b - a) + 1u;
-        return slabs & (((1u << n) - 1u) << min(a, b));
-    }
-
-    static __device__ __forceinline__ uint32_t med3(uint32_t v, uint32_t lo, uint32_t hi) { return min(max(v, lo), hi); }
-
-    // lanes in kDown: into the child block of the current cell
-    __device__ __forceinline__ void down_level(const WorldView& w)
-    {
-        WalkLds& l = walk_lds();
-        const bool top = s == 2u;  // at the top grid: the child is a brick
-        uint32_t slabs = ~0u;
-        if (top) slabs = w.proj[o & 0x3fffffu] | solid;
-        const uint32_t bits = top ? 3u : 2u;
-        const float scale = top ? 1.0f : 0.125f;  // map -> child cells
-        const float grow = top ? 8.0f : 4.0f;     // child cells per cell
-        const f3 As = f3{A.x * scale, A.y * scale, A.z * scale};
-        const float tc = t * grow;
-        const uint32_t first = (org + p) << bits;  // the child block's first cell
-        const uint32_t lx = first >> 20, ly = __builtin_amdgcn_ubfe(first, 10u, 10u), lz = first & 1023u;
-        const uint32_t n1 = top ? 7u : 3u;
-        const uint32_t cx = med3(f2u(As.x + V.x * tc), lx, lx + n1);
-        const uint32_t cy = med3(f2u(As.y + V.y * tc), ly, ly + n1);
-        const uint32_t cz = med3(f2u(As.z + V.z * tc), lz, lz + n1);
-        const float te = fminf(tx, fminf(ty, tz)) * grow;
-        const uint32_t ex = med3(f2u(__builtin_fmaf(V.x, te, As.x + copysignf(kSlack, V.x))), lx, lx + n1);
-        const uint32_t ey = med3(f2u(__builtin_fmaf(V.y, te, As.y + copysignf(kSlack, V.y))), ly, ly + n1);
-        const uint32_t ez = med3(f2u(__builtin_fmaf(V.z, te, As.z + copysignf(kSlack, V.z))), lz, lz + n1);
-        const uint32_t bx = slabs_between(slabs & 255u, cx - lx, ex - lx);
-        const uint32_t by = slabs_between((slabs >> 8) & 255u, cy - ly, ey - ly);
-        const uint32_t bz = slabs_between((slabs >> 16) & 255u, cz - lz, ez - lz);
-        const bool may = min(min(bx, by), bz) != 0u;
-        // the parent's state (unused at a brick that is left out)
-        const int k = top ? 1 : 0;
-        l.tx[k][threadIdx.x] = tx, l.ty[k][threadIdx.x] = ty, l.tz[k][threadIdx.x] = tz, l.p[k][threadIdx.x] = p;
-        if (top) l.base[threadIdx.x] = base;
-        const uint32_t child = top ? o << 9 : w.top + (cell(p, 5u) << 6);
-        steps += may ? 0 : cost;
-        t = may ? tc : t;
-        tx = may ? ((float)(cx + (V.x > 0 ? 1u : 0u)) - As.x) * rV.x : tx;
-        ty = may ? ((float)(cy + (V.y > 0 ? 1u : 0u)) - As.y) * rV.y : ty;
-        tz = may ? ((float)(cz + (V.z > 0 ? 1u : 0u)) - As.z) * rV.z : tz;
-        p = may ? ((cx - lx) << 20) | ((cy - ly) << 10) | (cz - lz) : p;
-        base = may ? child : base;
-        org = may ? first : org;
-        s = may ? bits : s;
-        outside = may ? (top ? kOut3 : kOut2) : outside;
-        cost = may ? (top ? 0 : 1) : cost;
-        o = 0u;
-        if (may) o = w.bricks[(size_t)(base + cell(p, s))];
-        mode = kStep;
-    }
-
-    __device__ __forceinline__ float distance() const { return (s == 3u ? t : t * 8.0f) + to; }
-
-    __device__ __forceinline__ uint64_t stepping() const { return __builtin_amdgcn_ballot_w64(mode == kStep); }
-    __device__ __forceinline__ uint64_t changing() const { return __builtin_amdgcn_ballot_w64(mode > kIdle); }
-    __device__ __forceinline__ bool more_steps() const { return (int)lanes(stepping()) - (int)lanes(changing()) > 0; }
-
-    // Step turns while more lanes have a cell to visit than a level to change.
+    // Step turns while more lanes have a cell to visit than a level to change:
+    // the lanes visit their cell (budget, solid cell or voxel, child block),
+    // then step to the next one.
     // A lane is in the brick it is in since before the run (only a change
     // turn enters one), and a brick walk that advances leaves within 22 steps
     // (7 per axis and the one that leaves).  A ray whose steps do not advance
@@ -570,19 +486,130 @@ struct Walk {
     // repeated were of one voxel, as in trace()'s 24.
     __device__ __forceinline__ void step_run(const WorldView& w)
     {
+        const uint64_t began = step_;
+        const uint64_t uber = lanes_where(cost == 4), grids = lanes_where(cost != 0);
         uint32_t n = 0u;
         if (more_steps()) do {
-            step(w);
+            steps -= lane_in(step_) ? cost : 0;
+            const uint64_t visit = step_ & ~lanes_where(steps <= 0);
+            const uint64_t child = visit & grids & lanes_where((int32_t)o < 0);
+            const uint64_t stops = visit & ~child & lanes_where(KIND == kTraceAll ? o != 0u : (o & 0xf000u) == 0xf000u);
+            const uint64_t go = visit & ~child & ~stops;
+            if (lane_in(go)) {
+                const float tn = fminf(tx, fminf(ty, tz));
+                const bool sx = tn == tx, sy = tn == ty, sz = tn == tz;
+                tx += sx ? fabsf(rV.x) : 0.0f;
+                ty += sy ? fabsf(rV.y) : 0.0f;
+                tz += sz ? fabsf(rV.z) : 0.0f;
+                p += (sx ? dx : 0u) + (sy ? dy : 0u) + (sz ? dz : 0u);
+                last = sz ? 2u : (sy ? 1u : 0u);
+                t = tn;
+            }
+            const uint64_t out = go & lanes_where((p & outside) != 0u);
+            down_ |= child, hit_ |= stops;
+            up_ |= ((step_ & ~visit) | out) & ~uber;
+            step_ = go & ~out;
+            if (lane_in(step_)) {
+                uint32_t at = word();
+                asm volatile("; step" : "+v"(at));  // keeps the load in this unit
+                o = w.bricks[(size_t)at];
+            }
             n++;
         } while (more_steps() && n < 32u);
-        if (n == 32u) mode = mode == kStep && s == 3u ? kUp : mode;
+        if (n == 32u) {
+            const uint64_t stuck = step_ & ~grids;
+            step_ &= ~stuck, up_ |= stuck;
+        }
+        // out of budget or out of the map at the uber level
+        miss_ |= began & ~(step_ | down_ | up_ | hit_);
     }
 
+    // one axis of the box test: the brick's slabs between local cells a and b
+    static __device__ __forceinline__ uint32_t slabs_between(uint32_t slabs, uint32_t a, uint32_t b)
+    {
+        const uint32_t n = (a > b ? a - b : b - a) + 1u, lo = min(a, b);
+        uint32_t m;  // n <= 8 bits from bit lo
+        asm("v_bfm_b32 %0, %1, %2" : "=v"(m) : "v"(n), "v"(lo));
+        return slabs & m;
+    }
+
+    // v clamped to [lo, hi] in one instruction
+    static __device__ __forceinline__ uint32_t med3(uint32_t v, uint32_t lo, uint32_t hi)
+    {
+        uint32_t m;
+        asm("v_med3_u32 %0, %1, %2, %3" : "=v"(m) : "v"(v), "v"(lo), "v"(hi));
+        return m;
+    }
+
+    // A change turn: every lane that has one changes its level.
     __device__ __forceinline__ void change(const WorldView& w)
     {
-        if (mode == kUp) up_level(w);
-        if (mode == kDown) down_level(w);
+        WalkLds& l = walk_lds();
+        const uint32_t tid = threadIdx.x;
+        if (lane_in(up_)) {
+            // back to the parent, whose pending step follows without another
+            // visit (an empty cell, its budget given back)
+            const bool brick = cost == 0;
+            const int k = brick ? 1 : 0;
+            tx = l.tx[k][tid], ty = l.ty[k][tid], tz = l.tz[k][tid], p = l.p[k][tid];
+            base = brick ? l.base[tid] : w.top + kTopWords;
+            org = brick ? l.org[tid] : 0u;
+            outside = brick ? kOut2 : kOut5, weights = brick ? kWeights2 : kWeights5, cost = brick ? 1 : 4;
+            dz = brick ? dz : dz << 3;
+            steps += cost, o = 0u;
+        }
+        if (lane_in(down_)) {
+            // into the child block of the current cell
+            const bool top = cost == 1;  // at the top grid: the child is a brick
+            uint32_t slabs = ~0u;
+            if (top) slabs = w.proj[o & 0x3fffffu];
+            slabs = lane_in(solid_) ? ~0u : slabs;
+            const uint32_t bits = top ? 3u : 2u, n1 = top ? 7u : 3u;
+            const float scale = top ? 1.0f : 0.125f;  // map -> child cells
+            const float grow = top ? 8.0f : 4.0f;     // child cells per cell
+            const f3 As = f3{A.x * scale, A.y * scale, A.z * scale};
+            const float tc = t * grow;
+            // the child block's first cell
+            const uint32_t z0 = (p >> 16) >> (top ? 0u : 3u);
+            const uint32_t lx = ((org >> 20) + (p & 255u)) << bits;
+            const uint32_t ly = (__builtin_amdgcn_ubfe(org, 10u, 10u) + __builtin_amdgcn_ubfe(p, 8u, 8u)) << bits;
+            const uint32_t lz = ((org & 1023u) + z0) << bits;
+            const uint32_t cx = med3(f2u(As.x + V.x * tc), lx, lx + n1);
+            const uint32_t cy = med3(f2u(As.y + V.y * tc), ly, ly + n1);
+            const uint32_t cz = med3(f2u(As.z + V.z * tc), lz, lz + n1);
+            const float te = fminf(tx, fminf(ty, tz)) * grow;
+            const uint32_t ex = med3(f2u(__builtin_fmaf(V.x, te, As.x + copysignf(kSlack, V.x))), lx, lx + n1);
+            const uint32_t ey = med3(f2u(__builtin_fmaf(V.y, te, As.y + copysignf(kSlack, V.y))), ly, ly + n1);
+            const uint32_t ez = med3(f2u(__builtin_fmaf(V.z, te, As.z + copysignf(kSlack, V.z))), lz, lz + n1);
+            const uint32_t bx = slabs_between(slabs, cx - lx, ex - lx);
+            const uint32_t by = slabs_between(slabs >> 8, cy - ly, ey - ly);
+            const uint32_t bz = slabs_between(slabs >> 16, cz - lz, ez - lz);
+            const bool may = min(min(bx, by), bz) != 0u;
+            // the parent's state (unused at a brick that is left out)
+            const int k = top ? 1 : 0;
+            l.tx[k][tid] = tx, l.ty[k][tid] = ty, l.tz[k][tid] = tz, l.p[k][tid] = p;
+            if (top) l.base[tid] = base, l.org[tid] = org;
+            const uint32_t child = top ? o << 9 : w.top + (__builtin_amdgcn_udot4(p, kWeights5, 0u, false) << 6);
+            steps += may ? 0 : cost;
+            t = may ? tc : t;
+            tx = may ? ((float)(cx + (V.x > 0 ? 1u : 0u)) - As.x) * rV.x : tx;
+            ty = may ? ((float)(cy + (V.y > 0 ? 1u : 0u)) - As.y) * rV.y : ty;
+            tz = may ? ((float)(cz + (V.z > 0 ? 1u : 0u)) - As.z) * rV.z : tz;
+            p = may ? (cx - lx) | ((cy - ly) << 8) | ((cz - lz) << 16) : p;
+            dz = may && !top ? (uint32_t)((int32_t)dz >> 3) : dz;
+            base = may ? child : base;
+            org = may ? (lx << 20) | (ly << 10) | lz : org;
+            outside = may ? (top ? kOut3 : kOut2) : outside;
+            weights = may ? (top ? kWeights3 : kWeights2) : weights;
+            cost = may ? (top ? 0 : 1) : cost;
+            o = 0u;
+            if (may) o = w.bricks[(size_t)word()];
+        }
+        step_ |= up_ | down_;
+        up_ = down_ = 0u;
     }
+
+    __device__ __forceinline__ float distance() const { return (cost == 0 ? t : t * 8.0f) + to; }
 };
 
 // A list of rays traced by waves that refill: a lane whose ray has ended
@@ -593,31 +620,35 @@ struct Walk {
 // so that the set-up of a ray runs for several lanes at a time (8, 24 and 32
 // free lanes were slower by 0.1-1%).  The MIS merge's rays of the moving
 // 1920x1080 scene: 0.95 -> 0.62 ms, 172 rays a wave, 56% of the lanes busy.
-// fetch(i, A, B): ray i's origin and direction, for this lane; finish(k):
-// the lane's ray has ended (k.mode kHit or kMiss).
-constexpr uint32_t kRefill = 16u;
+// fetch(i, A, B): ray i's origin and direction, for this lane; finish(hit,
+// k): the lane's ray has ended.
+constexpr int kRefill = 16;
 
 template <int KIND, class Fetch, class Finish>
 __device__ __forceinline__ void walk_list(const WorldView& w, int steps, uint32_t n, Fetch fetch, Finish finish)
 {
     Walk<KIND> k;
-    k.mode = kIdle;
+    k.clear();
     const uint32_t stride = gridDim.x * 256u;
     uint32_t cur = __builtin_amdgcn_readfirstlane(blockIdx.x * 256u + (threadIdx.x & ~63u));
     uint32_t end = min(cur + 64u, n);
     while (true) {
-        const uint64_t busy = k.stepping() | k.changing();
-        if (cur < n && 64u - lanes(busy) >= kRefill) {
-            if (k.mode == kHit || k.mode == kMiss) finish(k);
+        const uint64_t busy = k.step_ | k.down_ | k.up_;
+        if (cur < n && 64 - lanes(busy) >= kRefill) {
+            const bool hit = lane_in(k.hit_);
+            if (lane_in(k.hit_ | k.miss_)) finish(hit, k);
             const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(~busy >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)~busy, 0u));
-            const bool take = k.mode != kStep && k.mode <= kIdle && cur + rank < end;
-            if (k.mode == kHit || k.mode == kMiss) k.mode = kIdle;
+            const bool take = lane_in(~busy) && cur + rank < end;
+            bool alive = false, free_ = true;
             if (take) {
                 f3 A, B;
                 fetch(cur + rank, A, B);
-                k.begin(w, A, B, steps);
+                alive = k.begin(w, A, B, steps, free_);
             }
-            cur += lanes(~busy);
+            k.step_ |= lanes_where(alive);
+            k.hit_ = 0u, k.miss_ = lanes_where(take && !alive);
+            k.solid_ = (k.solid_ & busy) | lanes_where(!free_);
+            cur += (uint32_t)lanes(~busy);
             if (cur >= end) {
                 // the chunk's first ray, one grid further
                 const uint32_t first = end - 1u - ((end - 1u) & 63u);
@@ -630,20 +661,23 @@ __device__ __forceinline__ void walk_list(const WorldView& w, int steps, uint32_
         k.step_run(w);
         k.change(w);
     }
-    if (k.mode == kHit || k.mode == kMiss) finish(k);
+    const bool hit = lane_in(k.hit_);
+    if (lane_in(k.hit_ | k.miss_)) finish(hit, k);
 }
 
 template <int KIND>
 __device__ __forceinline__ uint32_t trace_free(const WorldView& w, f3 A, f3 B, int steps, float& dist, uint32_t& side)
 {
     Walk<KIND> k;
-    k.begin(w, A, B, steps);
-    while (true) {
+    k.clear();
+    bool free_;
+    k.step_ = lanes_where(k.begin(w, A, B, steps, free_));
+    k.solid_ = lanes_where(!free_);
+    while ((k.step_ | k.down_ | k.up_) != 0u) {
         k.step_run(w);
-        if ((k.stepping() | k.changing()) == 0u) break;
         k.change(w);
     }
-    if (k.mode != kHit) return 0u;
+    if (!lane_in(k.hit_)) return 0u;
     dist = k.distance(), side = k.last;
     return k.o;
 }

@@ -1183,11 +1183,11 @@ __global__ __launch_bounds__(256) VR_WAVES(8) void k_mis_trace(FrameArgs a, MisB
             l.d[t] = make_float4(r.L.x, r.L.y, r.L.z, __uint_as_float(task.x));
             A = r.spo, B = r.L;
         },
-        [&](const Walk<kTraceOpaque>& k) {
+        [&](bool hit, const Walk<kTraceOpaque>& k) {
             const float4 o = vload(l.o[t]), d = vload(l.d[t]);
             const uint32_t light = __float_as_uint(o.w), task = __float_as_uint(d.w);
             const float4 tla = a.L.a[light], tlb = a.L.b[light];
-            if (k.mode == kMiss || !hit_inside_light(k.last, k.distance(), __float_as_uint(tlb.w), (uint32_t)tla.w,
+            if (!hit || !hit_inside_light(k.last, k.distance(), __float_as_uint(tlb.w), (uint32_t)tla.w,
                                                      f3{o.x, o.y, o.z}, f3{d.x, d.y, d.z}))
                 atomicOr(&m.occ[task >> 5], 1u << (task & 31u));
         });
