@@ -101,6 +101,65 @@ __device__ __forceinline__ f3 normalize(f3 v)
 }
 
 // ---------------------------------------------------------------------------
+// Correctly rounded square root, reciprocal and quotient for operands of
+// middling size.  The general ones scale their operands, test for specials
+// and undo both again: 56 and 34 issue cycles of a SIMD (v_rsq and v_rcp take
+// 8, compares, selects and v_div_* 4, fma, mul and add 2) against 16, 12 and
+// 22 here.
+//   sqrt_mid(x)    x in [2^-100, 2^100): the estimate x*rsq(x) corrected by
+//                  its residual; equals sqrtf on every float of the range
+//                  (compared one by one on gfx950)
+//   rcp_mid(x)     |x| in [2^-100, 2^100): one Newton step from v_rcp_f32;
+//                  equals 1.0f/x on every float of the range (likewise)
+//   div_mid(a, b)  |b| in that range, a zero or |a| and |a/b| in it too: the
+//                  correctly rounded reciprocal and two residual steps, the
+//                  second of which rounds correctly (Markstein 1990: q within
+//                  one ulp of a/b and y = RN(1/b) give RN(q + y*(a - b*q)) =
+//                  RN(a/b))
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ float sqrt_mid(float x)
+{
+    const float y = __builtin_amdgcn_rsqf(x);
+    const float s = x * y;
+    return __builtin_fmaf(__builtin_fmaf(-s, s, x), 0.5f * y, s);
+}
+
+__device__ __forceinline__ float rcp_mid(float x)
+{
+    const float y = __builtin_amdgcn_rcpf(x);
+    return __builtin_fmaf(__builtin_fmaf(-x, y, 1.0f), y, y);
+}
+
+// a/b with y = RN(1/b)
+__device__ __forceinline__ float div_by(float a, float b, float y)
+{
+    float q = a * y;
+    q = __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
+    return __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
+}
+
+__device__ __forceinline__ float div_mid(float a, float b) { return div_by(a, b, rcp_mid(b)); }
+
+// x lies outside [2^kLo, 2^kHi] (or is not a number)
+template <int kLo, int kHi>
+__device__ __forceinline__ bool outside(float x)
+{
+    constexpr uint32_t lo = (uint32_t)(127 + kLo) << 23, hi = (uint32_t)(127 + kHi) << 23;
+    return __float_as_uint(x) - lo > hi - lo;
+}
+
+// any active lane of the wave (a scalar condition)
+__device__ __forceinline__ bool any_lane(bool b) { return __builtin_amdgcn_ballot_w64(b) != 0u; }
+
+// a/b, the mid-range way where every lane's operands allow it
+__device__ __forceinline__ float divide(float a, float b)
+{
+    float q = div_mid(a, b);
+    if (any_lane((a != 0.0f && outside<-60, 60>(a)) || outside<-40, 40>(b))) q = a / b;
+    return q;
+}
+
+// ---------------------------------------------------------------------------
 // RNG (cl/tools.cl:17-19)
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ uint32_t wang_hash(uint32_t s)
@@ -713,11 +772,40 @@ __device__ __forceinline__ f3 phat_full(bool point, f3 pos, f3 Nl, f3 sp, f3 N, 
     return f3{brdf.x * Le.x * NdotL * sa, brdf.y * Le.y * NdotL * sa, brdf.z * Le.z * NdotL * sa};
 }
 
-__device__ __forceinline__ float phat(bool point, f3 pos, f3 Nl, f3 sp, f3 N, f3 brdf, f3 Le, float size)
+// Length of a target vector; 0 when it is not finite
+__device__ __forceinline__ float phat_length(f3 v)
 {
-    const f3 v = phat_full(point, pos, Nl, sp, N, brdf, Le, size);
     const float r = sqrtf(dot(v, v));
     return (isnan(r) || isinf(r)) ? 0.0f : r;
+}
+
+// |phat_full| with the mid-range square roots and quotients; `odd` is set
+// when an operand lies outside their range and the value does not count.
+// nl: dot(Nl, -L) of a light face, given its axis's L; unused in point mode.
+template <class NlDotL>
+__device__ __forceinline__ float phat_mid(bool point, f3 pos, f3 sp, f3 N, f3 brdf, f3 Le, float size, NlDotL nl, bool& odd)
+{
+    const f3 R = sub(pos, sp);
+    const float d = dot(R, R);
+    const float inv = rcp_mid(sqrt_mid(d));
+    const f3 L = f3{R.x * inv, R.y * inv, R.z * inv};
+    const float NdotL = fmaxf(dot(N, L), 0.0f);
+    const float d2 = fmaxf(1e-5f, d);
+    const float area = size * size;
+    const float nldl = point ? 1.0f : fmaxf(nl(L), 0.0f);
+    const float sa = div_mid(nldl * area, d2);
+    const f3 v = f3{brdf.x * Le.x * NdotL * sa, brdf.y * Le.y * NdotL * sa, brdf.z * Le.z * NdotL * sa};
+    const float x = dot(v, v);
+    odd = outside<-80, 40>(d) || (x != 0.0f && outside<-96, 60>(x)) || (nldl != 0.0f && outside<-40, 1>(nldl));
+    return x == 0.0f ? 0.0f : sqrt_mid(x);
+}
+
+__device__ __forceinline__ float phat(bool point, f3 pos, f3 Nl, f3 sp, f3 N, f3 brdf, f3 Le, float size)
+{
+    bool odd;
+    float r = phat_mid(point, pos, sp, N, brdf, Le, size, [&](f3 L) { return dot(Nl, neg(L)); }, odd);
+    if (any_lane(odd)) r = phat_length(phat_full(point, pos, Nl, sp, N, brdf, Le, size));
+    return r;
 }
 
 // ---------------------------------------------------------------------------
@@ -731,14 +819,25 @@ struct Res {
     uint32_t face;  // Nlight as face index, 7 = zero vector
 };
 
-// true when the new sample takes the reservoir's place
+// UpdateReservoir's weight sum and decision (reservoir.cl:3-15): true when
+// the new sample takes the reservoir's place.  The quotient only decides a
+// comparison, so an estimate (within 2^-21 of it) serves unless r0 is that
+// close to it.
+__device__ __forceinline__ bool update_takes(float& wsum, float w, float r0)
+{
+    wsum += w;
+    const float m = fmaxf(1e-5f, wsum);
+    const float q = w * __builtin_amdgcn_rcpf(m);
+    bool take = r0 < q;
+    if (any_lane(!(fabsf(r0 - q) > q * 0x1p-20f && m < 0x1p100f))) take = r0 < w / m;
+    return take;
+}
+
 __device__ __forceinline__ bool res_update(Res& r, float w, float pHat, uint32_t index, float r0, f3 pos,
                                            float invPdf, uint32_t face)
 {
-    // UpdateReservoir (reservoir.cl:3-15)
     r.M += 1u;
-    r.wsum += w;
-    const bool take = r0 < w / fmaxf(1e-5f, r.wsum);
+    const bool take = update_takes(r.wsum, w, r0);
     if (take) {
         r.light = index, r.pos = pos, r.invPdf = invPdf, r.face = face, r.pHat = pHat;
     }

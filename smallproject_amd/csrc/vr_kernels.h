@@ -122,11 +122,12 @@ constexpr uint32_t kDdaScheduled = 0u, kDdaNested = 1u;
 // default occupancy targets (waves per SIMD) of the stage kernels: primary,
 // candidates, spatial reuse + shading.  The primary pass mostly runs beside
 // the previous frame's last stage, where fewer of its waves slow that stage
-// less (c2: 0.24 ms at 5 against 0.31 ms at 8, the same when alone); the
-// last stage then runs best at 8 (0.57 against 0.62 ms at 7, the same when
-// alone).  The MIS merge's variant holds its tile's ray list in LDS and more
+// less (c2: 0.24 ms at 5 against 0.31 ms at 8, the same when alone).  Whole
+// c2 frames: candidates at 5 / 6 / 7 waves 1.70 / 1.66 / 1.66 ms (6 spills
+// 2 registers, 7 spills 13), the last stage at 6 / 7 / 8 1.65 / 1.64 / 1.66
+// ms.  The MIS merge's variant holds its tile's ray list in LDS and more
 // live values, and runs best at 5.
-constexpr uint32_t kDefaultWaves[3] = {5, 7, 8};
+constexpr uint32_t kDefaultWaves[3] = {5, 6, 7};
 constexpr uint32_t kDefaultWavesMis = 5;
 // the split MIS merge's merge/list and weights/shading kernels (the tracer
 // runs at 8)
