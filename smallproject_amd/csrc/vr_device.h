@@ -49,10 +49,15 @@ __device__ __forceinline__ uint32_t brick_slabs(uint32_t x, uint32_t y, uint32_t
 // Light record prepared by the host from struct Light (common.h:134-139):
 // a = (centre.xyz, size), b = (Le.rgb, position bits).  Le is
 // ToFloatRGB(v) * EmitStrength(v) [* 1/pi with GFXEXP] as phat.cl:8-12
-// computes it per evaluation.
+// computes it per evaluation.  One 32-byte record, so that a light is one
+// cache line: candidates draw their lights at random, and every wave's 64
+// lights are 64 lines that L2 has to send to the compute unit's L1.
+struct Light {
+    float4 a, b;
+};
+
 struct LightView {
-    const float4* __restrict__ a;
-    const float4* __restrict__ b;
+    const Light* __restrict__ rec;
     // power source: bucket i of the alias table as (prob_i, alias_i bits,
     // pmf_i, pmf_alias_i), so one 16-byte load yields the light and its pdf;
     // null for the uniform source

@@ -10,8 +10,7 @@ constexpr uint32_t kNoTarget = 0xffffffffu;
 
 // the light records (as the render kernels read them) and the motion state
 struct LightMotionView {
-    float4* la;              // (centre.xyz, size)
-    float4* lb;              // (Le.rgb, packed position bits)
+    Light* lights;
     float4* pos;             // sub-voxel position (xyz)
     float4* vel;             // voxels per frame (xyz)
     const uint32_t* voxel;   // voxel word written at the light's voxel

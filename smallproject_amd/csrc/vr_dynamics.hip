@@ -100,8 +100,8 @@ __global__ __launch_bounds__(256) void k_light_claim(LightMotionView m, const ui
     const uint32_t i = blockIdx.x * 256u + threadIdx.x;
     if (i >= m.n) return;
     m.target[i] = kNoTarget;
-    if (m.la[i].w != 1.0f) return;
-    const uint32_t cur = __float_as_uint(m.lb[i].w);
+    if (m.lights[i].a.w != 1.0f) return;
+    const uint32_t cur = __float_as_uint(m.lights[i].b.w);
     const uint32_t cx = cur & 1023u, cz = (cur >> 10) & 1023u, cy = cur >> 20;
     const float4 p = m.pos[i], v = m.vel[i];
     const float nx = p.x + v.x, ny = p.y + v.y, nz = p.z + v.z;
@@ -131,7 +131,7 @@ __global__ __launch_bounds__(256) void k_light_move(LightMotionView m, const uin
     if (i >= m.n) return;
     const uint32_t t = m.target[i];
     if (t == kNoTarget) return;
-    const uint32_t cur = __float_as_uint(m.lb[i].w);
+    const uint32_t cur = __float_as_uint(m.lights[i].b.w);
     const uint32_t cx = cur & 1023u, cz = (cur >> 10) & 1023u, cy = cur >> 20;
     if (m.claim[claim_bucket(t)] != i) {
         bounce(m, i, cx, cy, cz);
@@ -145,9 +145,9 @@ __global__ __launch_bounds__(256) void k_light_move(LightMotionView m, const uin
     atomicOr(&proj[st >> 9], brick_slabs(tx & 7u, ty & 7u, tz & 7u));  // slabs only grow, as in k_edit_bricks
     const float4 p = m.pos[i], v = m.vel[i];
     m.pos[i] = make_float4(p.x + v.x, p.y + v.y, p.z + v.z, 0.0f);
-    m.la[i] = make_float4((float)tx + 0.5f, (float)ty + 0.5f, (float)tz + 0.5f, 1.0f);
-    const float4 b = m.lb[i];
-    m.lb[i] = make_float4(b.x, b.y, b.z, __uint_as_float(t));
+    m.lights[i].a = make_float4((float)tx + 0.5f, (float)ty + 0.5f, (float)tz + 0.5f, 1.0f);
+    const float4 b = m.lights[i].b;
+    m.lights[i].b = make_float4(b.x, b.y, b.z, __uint_as_float(t));
 }
 
 }  // namespace

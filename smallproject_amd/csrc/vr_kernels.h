@@ -31,6 +31,14 @@ constexpr uint32_t kTraced = 1u << 30, kVisible = 1u << 31;
 // ray counts of a frame (FrameArgs::rays, when counting is on)
 enum RayCount { kRaysPrimary = 0, kRaysCandidate = 1, kRaysShading = 2, kRaysMis = 3, kRayKinds = 4 };
 
+// Bucket j of a cluster's alias table: (prob bits, light j, light of alias j,
+// alias j local index) and the two lights' in-cluster shares pmf_i / P_c, in
+// 32 bytes, so one cache line yields the light and its pdf
+struct alignas(32) ClusterBucket {
+    uint4 pick;
+    float2 share;
+};
+
 // Everything one frame's kernels read, passed by value (kernarg segment).
 struct FrameArgs {
     WorldView w;
@@ -57,12 +65,7 @@ struct FrameArgs {
     // is drawn with the cluster's power alias table
     const uint2* candSlot;
     const uint32_t* clusterStart;  // [257] offsets into the cluster-ordered light list
-    // bucket j of the list (cluster c's buckets are clusterStart[c]..): the
-    // alias table's (prob bits, light j, light of alias j, alias j local
-    // index) and the two lights' in-cluster shares pmf_i / P_c, so one pair
-    // of loads yields the light and its pdf
-    const uint4* clusterPick;
-    const float2* clusterPickShare;
+    const ClusterBucket* clusterPick;  // bucket j of the list (cluster c's buckets are clusterStart[c]..)
 };
 
 // Tile order (block id -> 16x16 tile).  Workgroups are dealt round-robin to

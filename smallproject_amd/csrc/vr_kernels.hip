@@ -521,15 +521,15 @@ __device__ __forceinline__ void initial_px(const FrameArgs& a, int x, int y)
                 int32_t k = f2i(u * (float)cnt);
                 k = k < 0 ? 0 : (k > (int32_t)cnt - 1 ? (int32_t)cnt - 1 : k);
                 const float fr = u * (float)cnt - (float)k;
-                const uint4 e = a.clusterPick[c0 + k];
-                const float2 sh = a.clusterPickShare[c0 + k];
+                const uint4 e = a.clusterPick[c0 + k].pick;
+                const float2 sh = a.clusterPick[c0 + k].share;
                 const bool keep = fr < __uint_as_float(e.x);
                 li = keep ? e.y : e.z;
                 pr = mc * (keep ? sh.x : sh.y);
             } else {
                 li = pick_light(a.L, a.source, seed, pr);
             }
-            const float4 la = a.L.a[li], lb = a.L.b[li];
+            const float4 la = a.L.rec[li].a, lb = a.L.rec[li].b;
             f3 pos;
             float invPdf, ph;
             uint32_t face;
@@ -565,8 +565,8 @@ __device__ __forceinline__ void initial_px(const FrameArgs& a, int x, int y)
         if (wsum != 0.0f) {
             // with wsum == 0 the discard would leave W = wsum = 0 unchanged
             const uint32_t light = __float_as_uint(chosen.w);
-            const float4 lb = a.L.b[light];
-            const float4 la = a.L.a[light];
+            const float4 lb = a.L.rec[light].b;
+            const float4 la = a.L.rec[light].a;
             const f3 L = normalize(sub(f3{chosen.x, chosen.y, chosen.z}, spo));
             occ = light_occluded<kNested>(a.w, __float_as_uint(lb.w), (uint32_t)la.w, spo, L, a.shadowSteps);
             shadow = kTraced | (occ ? 0u : kVisible);
@@ -609,12 +609,12 @@ __device__ __forceinline__ void initial_px(const FrameArgs& a, int x, int y)
                     const uint4 p1 = a.A.r1[pi];
                     Res prev = res_from(p0, p1, make_float2(0.0f, 0.0f));  // wsum and pHat are recomputed below
                     if (prev.light < nL) {
-                        const float4 pa = a.L.a[prev.light], pb = a.L.b[prev.light];
+                        const float4 pa = a.L.rec[prev.light].a, pb = a.L.rec[prev.light].b;
                         const float pph = phat(a.point, prev.pos, face_normal(prev.face), s.sp, s.N, s.brdf,
                                                f3{pb.x, pb.y, pb.z}, pa.w) * prev.invPdf;
                         res_reweigh(prev, pph, pm);
                         if (res_combine(res, prev, rnd(seed))) shadow = 0u;  // the traced sample was replaced
-                        const float4 ra = a.L.a[res.light], rb = a.L.b[res.light];
+                        const float4 ra = a.L.rec[res.light].a, rb = a.L.rec[res.light].b;
                         const float rph = phat(a.point, res.pos, face_normal(res.face), s.sp, s.N, s.brdf,
                                                f3{rb.x, rb.y, rb.z}, ra.w) * res.invPdf;
                         res_adjust(res, rph);
@@ -694,7 +694,7 @@ __device__ __forceinline__ Merge spatial_merge(const FrameArgs& a, int x, int y)
             continue;
         Res nr = res_from(n0, n1, make_float2(0.0f, 0.0f));  // wsum and pHat: the reweigh recomputes them
         if (nr.light >= a.L.n) continue;
-        const float4 la = a.L.a[nr.light], lb = a.L.b[nr.light];
+        const float4 la = a.L.rec[nr.light].a, lb = a.L.rec[nr.light].b;
         const float ph = phat(a.point, nr.pos, face_normal(nr.face), s.sp, s.N, s.brdf, f3{lb.x, lb.y, lb.z}, la.w) *
                          nr.invPdf;
         res_reweigh(nr, ph, nr.M);
@@ -759,7 +759,7 @@ __device__ __forceinline__ float mis_weight_tile(const FrameArgs& a, int x, int 
     f3 Nl = f3{0.0f, 0.0f, 0.0f};
     float den = 0.0f, psel = 0.0f;
     if (need) {
-        la = a.L.a[res.light], lb = a.L.b[res.light];
+        la = a.L.rec[res.light].a, lb = a.L.rec[res.light].b;
         Nl = face_normal(res.face);
         const float p0 = phat(a.point, res.pos, Nl, g.s.sp, g.s.N, g.s.brdf, f3{lb.x, lb.y, lb.z}, la.w);
         den = (float)g.M0 * p0;
@@ -820,7 +820,7 @@ __device__ __forceinline__ float mis_weight_tile(const FrameArgs& a, int x, int 
             const Shading sh = shading_at(a, nx, ny, a.cur.hitw[ni], nd);
             const f3 spo = f3{sh.sp.x + 0.1f * sh.N.x, sh.sp.y + 0.1f * sh.N.y, sh.sp.z + 0.1f * sh.N.z};
             const f3 Ld = normalize(sub(f3{smp.x, smp.y, smp.z}, spo));
-            const float4 tla = a.L.a[light], tlb = a.L.b[light];
+            const float4 tla = a.L.rec[light].a, tlb = a.L.rec[light].b;
             if (light_occluded<kNested>(a.w, __float_as_uint(tlb.w), (uint32_t)tla.w, spo, Ld, a.shadowSteps))
                 atomicOr(&L.occluded[owner], 1u << (tk >> 8));
         }
@@ -900,7 +900,7 @@ __device__ __forceinline__ bool shade_px(const FrameArgs& a, int x, int y)
                 if (light < a.L.n) {
                     const f3 pos = f3{__uint_as_float(r1.x), __uint_as_float(r1.y), __uint_as_float(r1.z)};
                     const f3 spo = f3{s.sp.x + 0.1f * s.N.x, s.sp.y + 0.1f * s.N.y, s.sp.z + 0.1f * s.N.z};
-                    const float4 la = a.L.a[light], lb = a.L.b[light];
+                    const float4 la = a.L.rec[light].a, lb = a.L.rec[light].b;
                     const f3 L = normalize(sub(pos, spo));
                     // the final record's shadow bits: the candidate pass traced
                     // this very ray (its sample survived both merges)
@@ -923,7 +923,7 @@ __device__ __forceinline__ bool shade_px(const FrameArgs& a, int x, int y)
                         if (park) h = a.cur.hitw[i2];
                         const f3 sp = park ? f3{pp.x, pp.y, pp.z} : s.sp;
                         const uint4 q0 = a.A.r0[i2], q1 = a.A.r1[i2];
-                        const float4 qa = a.L.a[q1.w], qb = a.L.b[q1.w];
+                        const float4 qa = a.L.rec[q1.w].a, qb = a.L.rec[q1.w].b;
                         const float Wq = __uint_as_float(q0.z), invPdf = __uint_as_float(q0.w);
                         const f3 posq = f3{__uint_as_float(q1.x), __uint_as_float(q1.y), __uint_as_float(q1.z)};
                         const f3 inc = phat_full(a.point, posq, face_normal((q0.x >> 24) & 7u), sp, hit_normal(h),
@@ -1193,7 +1193,7 @@ __global__ __launch_bounds__(256) VR_WAVES(W) void k_mis_list(FrameArgs a, MisBu
         m.occ[idx] = 0u;
         need = g.merged && g.res.wsum > 0.0f && g.res.light < a.L.n;
         if (need) {
-            la = a.L.a[g.res.light], lb = a.L.b[g.res.light];
+            la = a.L.rec[g.res.light].a, lb = a.L.rec[g.res.light].b;
             Nl = face_normal(g.res.face);
             const size_t npx = (size_t)a.W * a.H;
             uint32_t rs = g.seed0;
@@ -1282,7 +1282,7 @@ __global__ __launch_bounds__(256) VR_WAVES(8) void k_mis_trace(FrameArgs a, MisB
         for (uint32_t t = blockIdx.x * 256u + threadIdx.x; t < n; t += gridDim.x * 256u) {
             const uint2 task = m.list[t];
             const MisRay r = mis_ray(a, task);
-            const float4 tla = a.L.a[r.light], tlb = a.L.b[r.light];
+            const float4 tla = a.L.rec[r.light].a, tlb = a.L.rec[r.light].b;
             if (light_occluded<true>(w, __float_as_uint(tlb.w), (uint32_t)tla.w, r.spo, r.L, a.shadowSteps))
                 atomicOr(&m.occ[task.x >> 5], 1u << (task.x & 31u));
         }
@@ -1302,7 +1302,7 @@ __global__ __launch_bounds__(256) VR_WAVES(8) void k_mis_trace(FrameArgs a, MisB
         [&](bool hit, const Walk<kTraceOpaque>& k) {
             const float4 o = vload(l.o[t]), d = vload(l.d[t]);
             const uint32_t light = __float_as_uint(o.w), task = __float_as_uint(d.w);
-            const float4 tla = a.L.a[light], tlb = a.L.b[light];
+            const float4 tla = a.L.rec[light].a, tlb = a.L.rec[light].b;
             if (!hit || !hit_inside_light(k.last, k.distance(), __float_as_uint(tlb.w), (uint32_t)tla.w,
                                                      f3{o.x, o.y, o.z}, f3{d.x, d.y, d.z}))
                 atomicOr(&m.occ[task >> 5], 1u << (task & 31u));
@@ -1332,7 +1332,7 @@ __global__ __launch_bounds__(256) VR_WAVES(W) void k_mis_finish(FrameArgs a, Mis
             if (res.wsum > 0.0f && res.light < b.L.n) {
                 const float dist = __uint_as_float(b.A.r0[idx].y);
                 const Shading s = shading_at(b, x, y, hitw, dist);
-                const float4 la = b.L.a[res.light], lb = b.L.b[res.light];
+                const float4 la = b.L.rec[res.light].a, lb = b.L.rec[res.light].b;
                 const f3 Nl = face_normal(res.face);
                 const float p0 = phat(b.point, res.pos, Nl, s.sp, s.N, s.brdf, f3{lb.x, lb.y, lb.z}, la.w);
                 float den = (float)info.w * p0;

@@ -101,8 +101,7 @@ struct vr_ctx {
     uint32_t* stageIds = nullptr;   // [VR_MAXCOMMITS]
     uint32_t* stageData = nullptr;  // [VR_MAXCOMMITS * 512]
     // lights
-    float4* la = nullptr;
-    float4* lb = nullptr;
+    Light* lights = nullptr;
     float4* pick = nullptr;  // power source's alias table (LightView::pick)
     uint32_t nLights = 0, lightCap = 0;
     float* emitLut = nullptr;
@@ -136,8 +135,7 @@ struct vr_ctx {
     uint32_t adamStep = 0;
     uint32_t* clusterStart = nullptr;   // [kMaxClusters + 1]
     uint32_t* clusterOf = nullptr;      // [lights]
-    uint4* clusterPick = nullptr;       // [lights] FrameArgs::clusterPick
-    float2* clusterPickShare = nullptr; // [lights] FrameArgs::clusterPickShare
+    ClusterBucket* clusterPick = nullptr;  // [lights] FrameArgs::clusterPick
     float* clusterPower = nullptr;      // [kMaxClusters] P_c
     float powerLow = 0.0f;              // sum of P_c over clusters with (c & 4) == 0
     float mix = 0.25f;                  // defensive mixture weight of the power source
@@ -349,7 +347,7 @@ FrameArgs frame_args(const vr_ctx* c, const vr_render_params* p)
     FrameArgs a;
     std::memset(&a, 0, sizeof(a));
     a.w = world_view(c);
-    a.L = LightView{c->la, c->lb, c->pick, p ? p->numberOfLights : 0u};
+    a.L = LightView{c->lights, c->pick, p ? p->numberOfLights : 0u};
     if (p) {
         a.cam.ox = p->oneOverRes[0], a.cam.oy = p->oneOverRes[1];
         a.cam.E = f3{p->E[0], p->E[1], p->E[2]};
@@ -388,7 +386,6 @@ FrameArgs frame_args(const vr_ctx* c, const vr_render_params* p)
     a.candSlot = c->candSlot;
     a.clusterStart = c->clusterStart;
     a.clusterPick = c->clusterPick;
-    a.clusterPickShare = c->clusterPickShare;
     return a;
 }
 
@@ -565,7 +562,7 @@ int vr_destroy(vr_ctx* c)
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     if (c->side) (void)hipStreamSynchronize(c->side);
     dfree(c->grid), dfree(c->uber), dfree(c->bricks), dfree(c->proj), dfree(c->stageIds), dfree(c->stageData);
-    dfree(c->la), dfree(c->lb), dfree(c->pick), dfree(c->emitLut), dfree(c->frame);
+    dfree(c->lights), dfree(c->pick), dfree(c->emitLut), dfree(c->frame);
     dfree(c->rays);
     for (int i = 0; i < 2; i++) {
         dfree(c->hitw[i]), dfree(c->dist[i]), dfree(c->seed[i]);
@@ -573,7 +570,7 @@ int vr_destroy(vr_ctx* c)
     }
     dfree(c->mlpP), dfree(c->mlpM), dfree(c->mlpV), dfree(c->mlpG);
     dfree(c->mlpW1b), dfree(c->mlpW2b), dfree(c->mlpW2Tb), dfree(c->mlpW3b), dfree(c->mlpW3Tb);
-    dfree(c->clusterStart), dfree(c->clusterOf), dfree(c->clusterPick), dfree(c->clusterPickShare);
+    dfree(c->clusterStart), dfree(c->clusterOf), dfree(c->clusterPick);
     dfree(c->clusterPower);
     dfree(c->candSlot);
     dfree(c->misList), dfree(c->misCount), dfree(c->misOcc), dfree(c->misInfo), dfree(c->misTerms);
@@ -627,19 +624,18 @@ int vr_set_lights(vr_ctx* c, const vr_light* lights, uint32_t n)
 {
     if (!c) return VR_ERR_ARG;
     if (n > 0 && !lights) return fail(c, VR_ERR_ARG, "vr_set_lights: null lights");
-    std::vector<float4> ha(n), hb(n);
+    std::vector<Light> rec(n);
     for (uint32_t i = 0; i < n; i++) {
         if (lights[i].position >= (1u << 30) || lights[i].size == 0 || lights[i].size > 1024)
             return fail(c, VR_ERR_ARG, "vr_set_lights: light " + std::to_string(i) + " out of range");
-        light_record(c->cfg, lights[i], ha[i], hb[i]);
+        light_record(c->cfg, lights[i], rec[i].a, rec[i].b);
     }
     HIPCHK(c, hipStreamSynchronize(c->stream));
     if (n > c->lightCap) {
-        dfree(c->la), dfree(c->lb), dfree(c->pick);
-        c->la = c->lb = c->pick = nullptr;
+        dfree(c->lights), dfree(c->pick);
+        c->lights = nullptr, c->pick = nullptr;
         const uint32_t cap = n * 2;
-        if (dalloc(&c->la, cap) != hipSuccess || dalloc(&c->lb, cap) != hipSuccess ||
-            dalloc(&c->pick, cap) != hipSuccess) {
+        if (dalloc(&c->lights, cap) != hipSuccess || dalloc(&c->pick, cap) != hipSuccess) {
             // the old list's buffers are gone: leave an empty list, so that
             // no later frame or step can reach the freed records
             c->lightCap = 0, c->nLights = 0, c->motionN = 0;
@@ -654,8 +650,7 @@ int vr_set_lights(vr_ctx* c, const vr_light* lights, uint32_t n)
     // the cluster tables describe the previous list, even at the same size
     c->clusteredLights = 0;
     if (n == 0) return VR_OK;
-    HIPCHK(c, hipMemcpyAsync(c->la, ha.data(), (size_t)n * 16, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipMemcpyAsync(c->lb, hb.data(), (size_t)n * 16, hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, hipMemcpyAsync(c->lights, rec.data(), (size_t)n * sizeof(Light), hipMemcpyHostToDevice, c->stream));
     if (c->cfg.source_pdf == VR_SOURCE_POWER) {
         std::vector<float> prob, pmf;
         std::vector<uint32_t> alias;
@@ -1073,25 +1068,23 @@ int vr_set_light_clusters(vr_ctx* c, const uint32_t* clusterOf, uint32_t nlights
     HIPCHK(c, hipStreamSynchronize(c->stream));
     // bucket j of cluster k (global index c0 + j): prob, its own light, its
     // alias's light and local index, and both lights' shares
-    std::vector<uint4> pick(nlights);
-    std::vector<float2> pickShare(nlights);
+    std::vector<ClusterBucket> pick(nlights);
     for (uint32_t k = 0; k < (uint32_t)kMaxClusters; k++) {
         const uint32_t c0 = start[k], cnt = start[k + 1] - c0;
         for (uint32_t j = 0; j < cnt; j++) {
             const uint32_t self = lights[c0 + j], other = lights[c0 + alias[c0 + j]];
             uint32_t pb;
             std::memcpy(&pb, &prob[c0 + j], 4);
-            pick[c0 + j] = make_uint4(pb, self, other, alias[c0 + j]);
-            pickShare[c0 + j] = make_float2(share[self], share[other]);
+            pick[c0 + j].pick = make_uint4(pb, self, other, alias[c0 + j]);
+            pick[c0 + j].share = make_float2(share[self], share[other]);
         }
     }
     if (nlights > c->clusterLightCap) {
-        dfree(c->clusterOf), dfree(c->clusterPick), dfree(c->clusterPickShare);
-        c->clusterOf = nullptr, c->clusterPick = nullptr, c->clusterPickShare = nullptr, c->clusterLightCap = 0;
+        dfree(c->clusterOf), dfree(c->clusterPick);
+        c->clusterOf = nullptr, c->clusterPick = nullptr, c->clusterLightCap = 0;
         // the old tables are gone: no frame may use them if this fails
         c->nclusters = 0, c->clusteredLights = 0;
-        if (dalloc(&c->clusterOf, nlights) != hipSuccess || dalloc(&c->clusterPick, nlights) != hipSuccess ||
-            dalloc(&c->clusterPickShare, nlights) != hipSuccess)
+        if (dalloc(&c->clusterOf, nlights) != hipSuccess || dalloc(&c->clusterPick, nlights) != hipSuccess)
             return fail(c, VR_ERR_NOMEM, "vr_set_light_clusters: allocation failed");
         c->clusterLightCap = nlights;
     }
@@ -1099,9 +1092,8 @@ int vr_set_light_clusters(vr_ctx* c, const uint32_t* clusterOf, uint32_t nlights
     HIPCHK(c, hipMemcpyAsync(c->clusterPower, power.data(), kMaxClusters * 4, hipMemcpyHostToDevice, c->stream));
     if (nlights) {
         HIPCHK(c, hipMemcpyAsync(c->clusterOf, clusterOf, (size_t)nlights * 4, hipMemcpyHostToDevice, c->stream));
-        HIPCHK(c, hipMemcpyAsync(c->clusterPick, pick.data(), (size_t)nlights * 16, hipMemcpyHostToDevice, c->stream));
-        HIPCHK(c, hipMemcpyAsync(c->clusterPickShare, pickShare.data(), (size_t)nlights * 8, hipMemcpyHostToDevice,
-                                 c->stream));
+        HIPCHK(c, hipMemcpyAsync(c->clusterPick, pick.data(), (size_t)nlights * sizeof(ClusterBucket),
+                                 hipMemcpyHostToDevice, c->stream));
     }
     HIPCHK(c, hipStreamSynchronize(c->stream));
     c->powerLow = (float)low;
@@ -1138,15 +1130,14 @@ int vr_read_cluster_tables(vr_ctx* c, uint32_t* start, uint32_t* lights, float* 
     if (power) HIPCHK(c, hipMemcpy(power, c->clusterPower, kMaxClusters * 4, hipMemcpyDeviceToHost));
     if (n == 0) return VR_OK;
     // the tables as the kernels read them, unpacked
-    std::vector<uint4> pick(n);
-    std::vector<float2> pickShare(n);
-    HIPCHK(c, hipMemcpy(pick.data(), c->clusterPick, n * 16, hipMemcpyDeviceToHost));
-    HIPCHK(c, hipMemcpy(pickShare.data(), c->clusterPickShare, n * 8, hipMemcpyDeviceToHost));
+    std::vector<ClusterBucket> bucket(n);
+    HIPCHK(c, hipMemcpy(bucket.data(), c->clusterPick, n * sizeof(ClusterBucket), hipMemcpyDeviceToHost));
     for (size_t j = 0; j < n; j++) {
-        if (lights) lights[j] = pick[j].y;
-        if (prob) std::memcpy(&prob[j], &pick[j].x, 4);
-        if (alias) alias[j] = pick[j].w;
-        if (share && pick[j].y < n) share[pick[j].y] = pickShare[j].x;
+        const uint4 pick = bucket[j].pick;
+        if (lights) lights[j] = pick.y;
+        if (prob) std::memcpy(&prob[j], &pick.x, 4);
+        if (alias) alias[j] = pick.w;
+        if (share && pick.y < n) share[pick.y] = bucket[j].share.x;
     }
     return VR_OK;
 }
@@ -1363,7 +1354,8 @@ int vr_set_light_motion(vr_ctx* c, const float* velocity, uint32_t n)
     c->motionN = n;
     if (n == 0) return VR_OK;
     // positions start at the voxel centres the light records hold
-    HIPCHK(c, hipMemcpyAsync(c->lightPos, c->la, (size_t)n * 16, hipMemcpyDeviceToDevice, c->stream));
+    HIPCHK(c, hipMemcpy2DAsync(c->lightPos, sizeof(float4), &c->lights->a, sizeof(Light), sizeof(float4), n,
+                               hipMemcpyDeviceToDevice, c->stream));
     HIPCHK(c, hipMemcpyAsync(c->lightVel, vel.data(), (size_t)n * 16, hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipMemcpyAsync(c->lightVoxel, vox.data(), (size_t)n * 4, hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -1382,7 +1374,7 @@ int vr_scene_step(vr_ctx* c, uint32_t frame, uint32_t seed, uint32_t edit_permil
     c->worldEpoch++;  // the next primary pass waits for these edits
     HIPCHK(c, launch_edit_bricks(c->bricks, c->proj, high_water, frame, seed, edit_permille, walk_steps, c->stream));
     if (c->motionN > 0 && c->motionN == c->nLights) {
-        const LightMotionView m{c->la, c->lb, c->lightPos, c->lightVel, c->lightVoxel, c->lightTarget, c->claim,
+        const LightMotionView m{c->lights, c->lightPos, c->lightVel, c->lightVoxel, c->lightTarget, c->claim,
                                 c->motionN};
         HIPCHK(c, launch_move_lights(m, c->grid, c->bricks, c->proj, c->cfg.brick_capacity, c->stream));
     }
@@ -1394,13 +1386,13 @@ int vr_read_lights(vr_ctx* c, vr_light* out, uint32_t n)
     if (!c || (n > 0 && !out)) return VR_ERR_ARG;
     if (n != c->nLights) return fail(c, VR_ERR_ARG, "vr_read_lights: n must equal the light count");
     if (n == 0) return VR_OK;
-    std::vector<float4> lb(n);
-    HIPCHK(c, hipMemcpyAsync(lb.data(), c->lb, (size_t)n * 16, hipMemcpyDeviceToHost, c->stream));
+    std::vector<Light> rec(n);
+    HIPCHK(c, hipMemcpyAsync(rec.data(), c->lights, (size_t)n * sizeof(Light), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     for (uint32_t i = 0; i < n; i++) {
         out[i] = c->hostLights[i];
         uint32_t packed;
-        std::memcpy(&packed, &lb[i].w, 4);
+        std::memcpy(&packed, &rec[i].b.w, 4);
         const uint32_t x = packed & 1023u, z = (packed >> 10) & 1023u, y = packed >> 20;
         out[i].position = x + z * 1024u + y * 1024u * 1024u;
     }
