@@ -153,14 +153,26 @@ __device__ __forceinline__ bool outside(float x)
     return __float_as_uint(x) - lo > hi - lo;
 }
 
-// any active lane of the wave (a scalar condition)
-__device__ __forceinline__ bool any_lane(bool b) { return __builtin_amdgcn_ballot_w64(b) != 0u; }
+// Lane masks: conditions of the wave's lanes as a scalar word.  Conditions
+// that decide for the whole wave are combined as masks: a combination of
+// bools costs two vector instructions more to turn into one.
+__device__ __forceinline__ uint64_t lanes_where(bool b) { return __builtin_amdgcn_ballot_w64(b); }
+__device__ __forceinline__ bool lane_in(uint64_t mask) { return __builtin_amdgcn_inverse_ballot_w64(mask); }
 
-// a/b, the mid-range way where every lane's operands allow it
-__device__ __forceinline__ float divide(float a, float b)
+// a quotient that only rare lanes need: the compiler, left to itself, computes
+// it beside the short form on every call and selects (55 issue cycles)
+__device__ __forceinline__ float rare_quotient(float a, float b)
 {
-    float q = div_mid(a, b);
-    if (any_lane((a != 0.0f && outside<-60, 60>(a)) || outside<-40, 40>(b))) q = a / b;
+    asm volatile("" : "+v"(a), "+v"(b));
+    return a / b;
+}
+
+// a/b with y = RN(1/b), the mid-range way where every lane's operands allow it
+__device__ __forceinline__ float divide_by(float a, float b, float y)
+{
+    float q = div_by(a, b, y);
+    if (((lanes_where(a != 0.0f) & lanes_where(outside<-60, 60>(a))) | lanes_where(outside<-40, 40>(b))) != 0u)
+        q = rare_quotient(a, b);
     return q;
 }
 
@@ -443,8 +455,6 @@ __device__ __forceinline__ int lanes(uint64_t mask)
     asm("s_bcnt1_i32_b64 %0, %1" : "=s"(n) : "s"(mask) : "scc");
     return n;
 }
-__device__ __forceinline__ uint64_t lanes_where(bool b) { return __builtin_amdgcn_ballot_w64(b); }
-__device__ __forceinline__ bool lane_in(uint64_t mask) { return __builtin_amdgcn_inverse_ballot_w64(mask); }
 
 // Parent levels' state of the workgroup's lanes (256 threads at most): the
 // uber cell's and the top cell's crossing distances and packed cell, and the
@@ -784,11 +794,11 @@ __device__ __forceinline__ float phat_length(f3 v)
     return (isnan(r) || isinf(r)) ? 0.0f : r;
 }
 
-// |phat_full| with the mid-range square roots and quotients; `odd` is set
-// when an operand lies outside their range and the value does not count.
+// |phat_full| with the mid-range square roots and quotients; `odd`: the lanes
+// with an operand outside their range, whose value does not count.
 // nl: dot(Nl, -L) of a light face, given its axis's L; unused in point mode.
 template <class NlDotL>
-__device__ __forceinline__ float phat_mid(bool point, f3 pos, f3 sp, f3 N, f3 brdf, f3 Le, float size, NlDotL nl, bool& odd)
+__device__ __forceinline__ float phat_mid(bool point, f3 pos, f3 sp, f3 N, f3 brdf, f3 Le, float size, NlDotL nl, uint64_t& odd)
 {
     const f3 R = sub(pos, sp);
     const float d = dot(R, R);
@@ -801,15 +811,17 @@ __device__ __forceinline__ float phat_mid(bool point, f3 pos, f3 sp, f3 N, f3 br
     const float sa = div_mid(nldl * area, d2);
     const f3 v = f3{brdf.x * Le.x * NdotL * sa, brdf.y * Le.y * NdotL * sa, brdf.z * Le.z * NdotL * sa};
     const float x = dot(v, v);
-    odd = outside<-80, 40>(d) || (x != 0.0f && outside<-96, 60>(x)) || (nldl != 0.0f && outside<-40, 1>(nldl));
-    return x == 0.0f ? 0.0f : sqrt_mid(x);
+    const uint64_t some = lanes_where(x != 0.0f);
+    odd = lanes_where(outside<-80, 40>(d)) | (some & lanes_where(outside<-96, 60>(x))) |
+          (lanes_where(nldl != 0.0f) & lanes_where(outside<-40, 1>(nldl)));
+    return lane_in(some) ? sqrt_mid(x) : 0.0f;
 }
 
 __device__ __forceinline__ float phat(bool point, f3 pos, f3 Nl, f3 sp, f3 N, f3 brdf, f3 Le, float size)
 {
-    bool odd;
+    uint64_t odd;
     float r = phat_mid(point, pos, sp, N, brdf, Le, size, [&](f3 L) { return dot(Nl, neg(L)); }, odd);
-    if (any_lane(odd)) r = phat_length(phat_full(point, pos, Nl, sp, N, brdf, Le, size));
+    if (odd != 0u) r = phat_length(phat_full(point, pos, Nl, sp, N, brdf, Le, size));
     return r;
 }
 
@@ -834,7 +846,8 @@ __device__ __forceinline__ bool update_takes(float& wsum, float w, float r0)
     const float m = fmaxf(1e-5f, wsum);
     const float q = w * __builtin_amdgcn_rcpf(m);
     bool take = r0 < q;
-    if (any_lane(!(fabsf(r0 - q) > q * 0x1p-20f && m < 0x1p100f))) take = r0 < w / m;
+    if ((lanes_where(!(fabsf(r0 - q) > q * 0x1p-20f)) | lanes_where(!(m < 0x1p100f))) != 0u)
+        take = r0 < rare_quotient(w, m);
     return take;
 }
 

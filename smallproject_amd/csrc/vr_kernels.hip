@@ -259,31 +259,35 @@ __device__ __forceinline__ void point_on_voxel(f3 c, float size, f3 sp, uint32_t
 //   - A face's ndl is |R_a| / |R| (the face looks at the point), so the sign
 //     products and the clamp at 0 fall away exactly.
 //   - dot(Nl, -L) of an axis normal is -+L_a.
-// Returns false when some step lies outside what that covers (a comparison
-// closer than 2^-20, operands outside the mid range, no face that looks at
-// the point): the values do not count, and the caller takes point_on_voxel.
-// Both draw the same 13 numbers.  k_initial is bound by the issue of its
-// vector instructions: 26.8k -> 21.3k a wave, 1.18 -> 0.99 ms on c2 at
-// 1920x1080 with phat's and the reservoir update's short forms.
+//   - A sign (s = 1 for a +face) enters as a factor, which is exact; drawn
+//     coordinates are the drawn word times size/2^32 (likewise).
+// Returns the lanes for which some step lies outside what that covers (a
+// comparison closer than 2^-20, operands outside the mid range, no face that
+// looks at the point): their values do not count, and the caller takes
+// point_on_voxel.  Both draw the same 13 numbers.  k_initial is bound by the
+// issue of its vector instructions: 26.8k -> 21.3k a wave, 1.18 -> 0.99 ms on
+// c2 at 1920x1080 with phat's and the reservoir update's short forms.  What
+// an instruction costs a SIMD (gfx950, measured): 2 cycles for mul, add, xor,
+// right shifts and an fma of two registers, 4 for most others (fma of three,
+// selects, compares, left shifts, min/max, conversions), 8 for rcp and rsq;
+// a select by vcc in its short encoding right after another one 23.
 struct AreaSample {
     f3 pos;
     float invPdf, ph;
     uint32_t face;
 };
 
-__device__ __forceinline__ bool area_candidate(f3 c, float size, f3 spo, const f3& sp, const f3& N, const f3& brdf,
+__device__ __forceinline__ uint64_t area_candidate(f3 c, float size, f3 spo, const f3& sp, const f3& N, const f3& brdf,
                                                f3 Le, uint32_t& seed, AreaSample& o)
 {
-    const float hs = 0.5f * size;
+    const float hs = 0.5f * size, draw = size * 0x1p-32f;
     const float area = size * size;
     const float cc[3] = {c.x, c.y, c.z}, ss[3] = {spo.x, spo.y, spo.z};
-    float lo[3], hi[3];
-    bool plus[3], front[3];
+    uint64_t plus[3], front[3];
 #pragma unroll
     for (int a = 0; a < 3; a++) {
-        lo[a] = cc[a] - hs, hi[a] = cc[a] + hs;
-        plus[a] = hi[a] - ss[a] < 0.0f;
-        front[a] = plus[a] || lo[a] - ss[a] > 0.0f;
+        plus[a] = lanes_where((cc[a] + hs) - ss[a] < 0.0f);
+        front[a] = plus[a] | lanes_where((cc[a] - hs) - ss[a] > 0.0f);
     }
     uint32_t w0[3], w1[3];
 #pragma unroll
@@ -291,61 +295,70 @@ __device__ __forceinline__ bool area_candidate(f3 c, float size, f3 spo, const f
         const uint32_t v0 = xorshift(seed), v1 = xorshift(seed);
         const int a = k % 3;
         if (k < 3) w0[a] = v0, w1[a] = v1;
-        else w0[a] = plus[a] ? w0[a] : v0, w1[a] = plus[a] ? w1[a] : v1;
+        else w0[a] = lane_in(plus[a]) ? w0[a] : v0, w1[a] = lane_in(plus[a]) ? w1[a] : v1;
     }
     const float r2 = rnd(seed);
-    float sol[3];
+    float sol[3], dist2[3];
     f3 fp[3];
-    bool odd = false;
 #pragma unroll
     for (int a = 0; a < 3; a++) {
         const int t = (a + 1) % 3, b = (a + 2) % 3;
-        const float s0 = (float)w0[a] * 2.3283064365387e-10f * size, s1 = (float)w1[a] * 2.3283064365387e-10f * size;
+        const float s = lane_in(plus[a]) ? 1.0f : -1.0f;
+        const float hss = hs * s, ds = draw * s;
         float f[3];
-        f[a] = plus[a] ? hi[a] : lo[a];
-        f[t] = (plus[a] ? lo[t] : hi[t]) + (plus[a] ? s0 : -s0);
-        f[b] = (plus[a] ? lo[b] : hi[b]) + (plus[a] ? s1 : -s1);
+        f[a] = cc[a] + hss;
+        f[t] = (cc[t] - hss) + (float)w0[a] * ds;
+        f[b] = (cc[b] - hss) + (float)w1[a] * ds;
         fp[a] = f3{f[0], f[1], f[2]};
         const f3 R = sub(fp[a], spo);
         const float d = dot(R, R);
         const float Ra = a == 0 ? R.x : (a == 1 ? R.y : R.z);
         const float ndl = fabsf(Ra) * rcp_mid(sqrt_mid(d));
         const float q = div_mid(ndl * area, fmaxf(1e-5f, d));
-        sol[a] = front[a] ? q : 0.0f;
-        odd = odd || outside<-80, 40>(d);
+        sol[a] = lane_in(front[a]) ? q : 0.0f;
+        dist2[a] = d;
     }
-    // partial sums in face order: +x +y +z -x -y -z
+    uint64_t odd = lanes_where(outside<-80, 40>(dist2[0])) | lanes_where(outside<-80, 40>(dist2[1])) |
+                   lanes_where(outside<-80, 40>(dist2[2]));
+    // partial sums in face order: +x +y +z -x -y -z (a face's solid angle
+    // counts once: what the +face has not, the -face has)
     float cum[6], total = 0.0f;
 #pragma unroll
-    for (int k = 0; k < 6; k++) {
-        total += plus[k % 3] == (k < 3) ? sol[k % 3] : 0.0f;
+    for (int k = 0; k < 3; k++) {
+        cum[3 + k] = lane_in(plus[k]) ? sol[k] : 0.0f;
+        total += cum[3 + k];
+        cum[k] = total;
+    }
+#pragma unroll
+    for (int k = 3; k < 6; k++) {
+        total += sol[k - 3] - cum[k];
         cum[k] = total;
     }
     const float want = r2 * total;
     float gap = fabsf(total - want);
-    bool at[5];
+    uint64_t at[5];
 #pragma unroll
     for (int k = 0; k < 5; k++) {
         gap = fminf(gap, fabsf(cum[k] - want));
-        at[k] = cum[k] >= want;
+        at[k] = lanes_where(cum[k] >= want);
     }
-    odd = odd || !(gap > total * 0x1p-20f && total > 0x1p-60f);
+    odd |= lanes_where(!(gap > total * 0x1p-20f)) | lanes_where(!(total > 0x1p-60f));
     // the chosen face: the first whose partial sum reaches r2*total
-    const bool isX = at[0] || (at[3] && !at[2]), isY = (at[1] && !at[0]) || (at[4] && !at[3]);
-    const bool minus = !at[2];
+    const uint64_t onX = at[0] | (at[3] & ~at[2]), onY = (at[1] & ~at[0]) | (at[4] & ~at[3]);
+    const bool isX = lane_in(onX), isY = lane_in(onY), minus = lane_in(~at[2]);
     const float pick = isX ? sol[0] : (isY ? sol[1] : sol[2]);
     o.pos.x = isX ? fp[0].x : (isY ? fp[1].x : fp[2].x);
     o.pos.y = isX ? fp[0].y : (isY ? fp[1].y : fp[2].y);
     o.pos.z = isX ? fp[0].z : (isY ? fp[1].z : fp[2].z);
     o.face = (isX ? 0u : (isY ? 1u : 2u)) + (minus ? 3u : 0u);
     o.invPdf = rcp_mid(div_mid(pick, total));
-    bool odd2;
+    uint64_t odd2;
     const float ph = phat_mid(false, o.pos, sp, N, brdf, Le, size, [&](f3 L) {
         const float La = isX ? L.x : (isY ? L.y : L.z);
         return minus ? La : -La;
     }, odd2);
     o.ph = ph * o.invPdf;
-    return !(odd || odd2);
+    return odd | odd2;
 }
 
 __device__ __forceinline__ uint32_t pick_light(const LightView& L, uint32_t source, uint32_t& seed, float& p)
@@ -501,8 +514,10 @@ __device__ __forceinline__ void initial_px(const FrameArgs& a, int x, int y)
         pk.pos[t] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         pk.val[t] = make_float4(0.0f, 0.0f, __uint_as_float(7u), 0.0f);
         float wsum = 0.0f;
+        // RN(1/pdf) of the uniform source, in a scalar register
+        const float uniformRcp = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(rcp_mid(1.0f / (float)nL))));
         for (uint32_t i = 0; i < nC; i++) {
-            float pr;
+            float pr, prRcp;
             uint32_t li;
             if (a.source == 2u) {
                 // learned proposal: the slot's cluster and mixture mass; the
@@ -526,8 +541,11 @@ __device__ __forceinline__ void initial_px(const FrameArgs& a, int x, int y)
                 const bool keep = fr < __uint_as_float(e.x);
                 li = keep ? e.y : e.z;
                 pr = mc * (keep ? sh.x : sh.y);
+                prRcp = rcp_mid(pr);
             } else {
                 li = pick_light(a.L, a.source, seed, pr);
+                prRcp = uniformRcp;
+                if (a.source == 1u) prRcp = rcp_mid(pr);
             }
             const float4 la = a.L.rec[li].a, lb = a.L.rec[li].b;
             f3 pos;
@@ -539,16 +557,16 @@ __device__ __forceinline__ void initial_px(const FrameArgs& a, int x, int y)
             } else {
                 const uint32_t start = seed;
                 AreaSample as;
-                const bool mid = area_candidate(f3{la.x, la.y, la.z}, la.w, spo, s.sp, s.N, s.brdf,
-                                                f3{lb.x, lb.y, lb.z}, seed, as);
+                const uint64_t odd = area_candidate(f3{la.x, la.y, la.z}, la.w, spo, s.sp, s.N, s.brdf,
+                                                    f3{lb.x, lb.y, lb.z}, seed, as);
                 pos = as.pos, invPdf = as.invPdf, face = as.face, ph = as.ph;
-                if (any_lane(!mid)) {
+                if (odd != 0u) {
                     seed = start;
                     point_on_voxel(f3{la.x, la.y, la.z}, la.w, spo, seed, pos, invPdf, face);
                     ph = phat_length(phat_full(false, pos, face_normal(face), s.sp, s.N, s.brdf, f3{lb.x, lb.y, lb.z}, la.w)) * invPdf;
                 }
             }
-            if (update_takes(wsum, divide(ph, pr), rnd(seed))) {
+            if (update_takes(wsum, divide_by(ph, pr, prRcp), rnd(seed))) {
                 pk.pos[t] = make_float4(pos.x, pos.y, pos.z, __uint_as_float(li));
                 pk.val[t] = make_float4(ph, invPdf, __uint_as_float(face), 0.0f);
             }
