@@ -10,16 +10,19 @@ struct HitPlanes {
     uint32_t* seed;
 };
 
-// A plane of per-pixel reservoirs, as three structure-of-arrays records.
-// r0 holds what a reuse pass tests before it takes a reservoir, so a
-// neighbour or the previous frame's pixel that fails the tests costs one
-// 16-byte read: {M (bits 0-23) | Nlight face << 24 | the pixel's hit side
-// bits << 27 (side and the sign of D[side], bits 24-26 of the hit word) |
+// A plane of per-pixel reservoirs.  r0 holds what a reuse pass tests before
+// it takes a reservoir: {M (bits 0-23) | Nlight face << 24 | the pixel's hit
+// side bits << 27 (side and the sign of D[side], bits 24-26 of the hit word) |
 // kTraced | kVisible, hit distance, W, invPdf}.  r1 is the sample {pos.xyz,
-// light index}, r2 the sums {wsum, pHat}.
+// light index}, r2 the sums {wsum, pHat}.  A reuse pass reads r0 and r1 of
+// pixels scattered over a disc, so the two lie in one 32-byte record: one
+// cache line a pixel.  r2 is read by the pixel's own passes only.
+struct Record {
+    uint4 r0, r1;
+};
+
 struct ResPlanes {
-    uint4* r0;
-    uint4* r1;
+    Record* rec;
     float2* r2;
 };
 // r0.x bits 30-31: the candidate pass traced the shadow ray of this

@@ -38,7 +38,7 @@ __device__ __forceinline__ Res res_from(const uint4 r0, const uint4 r1, const fl
     return o;
 }
 
-__device__ __forceinline__ Res load_res(const ResPlanes& r, size_t i) { return res_from(r.r0[i], r.r1[i], r.r2[i]); }
+__device__ __forceinline__ Res load_res(const ResPlanes& r, size_t i) { return res_from(r.rec[i].r0, r.rec[i].r1, r.r2[i]); }
 
 // A neighbour's or the previous frame's record (r0) and sample (r1), loaded
 // together.  Its tests read the record word, then the distance, and only a
@@ -49,8 +49,8 @@ __device__ __forceinline__ Res load_res(const ResPlanes& r, size_t i) { return r
 // tests (spatial reuse: 0.565 -> 0.555 ms at 1080p).
 __device__ __forceinline__ void load_record_sample(const ResPlanes& r, size_t i, uint4& r0, uint4& r1)
 {
-    uint4 s = r.r1[i];
-    uint4 c = r.r0[i];
+    uint4 s = r.rec[i].r1;
+    uint4 c = r.rec[i].r0;
     asm volatile("" : "+v"(c.x), "+v"(c.y), "+v"(c.z), "+v"(c.w), "+v"(s.x), "+v"(s.y), "+v"(s.z), "+v"(s.w));
     r0 = c, r1 = s;
 }
@@ -60,9 +60,9 @@ __device__ __forceinline__ void load_record_sample(const ResPlanes& r, size_t i,
 __device__ __forceinline__ void store_res(const ResPlanes& r, size_t i, const Res& o, uint32_t hitw, float dist,
                                           uint32_t shadow)
 {
-    r.r0[i] = make_uint4((o.M & 0xffffffu) | ((o.face & 7u) << 24) | (((hitw >> 24) & 7u) << 27) | shadow,
+    r.rec[i].r0 = make_uint4((o.M & 0xffffffu) | ((o.face & 7u) << 24) | (((hitw >> 24) & 7u) << 27) | shadow,
                          __float_as_uint(dist), __float_as_uint(o.W), __float_as_uint(o.invPdf));
-    r.r1[i] = make_uint4(__float_as_uint(o.pos.x), __float_as_uint(o.pos.y), __float_as_uint(o.pos.z), o.light);
+    r.rec[i].r1 = make_uint4(__float_as_uint(o.pos.x), __float_as_uint(o.pos.y), __float_as_uint(o.pos.z), o.light);
     r.r2[i] = make_float2(o.wsum, o.pHat);
 }
 
@@ -618,13 +618,13 @@ __device__ __forceinline__ void initial_px(const FrameArgs& a, int x, int y)
                 // pixel: its record word and distance carry that pixel's
                 // hit (the previous hit buffer's side bits and distance)
                 const size_t pi = (size_t)py * a.W + px;
-                const uint4 p0 = a.A.r0[pi];
+                const uint4 p0 = a.A.rec[pi].r0;
                 const float pd = __uint_as_float(p0.y);
                 const uint32_t prevM = p0.x & 0xffffffu;
                 const uint32_t cap = a.maxTemporal * nC;
                 const uint32_t pm = cap < prevM ? cap : prevM;
                 if (same_face(rec_hit_bits(p0.x), hitw, a.axisOnlyFace) && fabsf(dist - pd) <= 0.1f * dist && pm > 0u) {
-                    const uint4 p1 = a.A.r1[pi];
+                    const uint4 p1 = a.A.rec[pi].r1;
                     Res prev = res_from(p0, p1, make_float2(0.0f, 0.0f));  // wsum and pHat are recomputed below
                     if (prev.light < nL) {
                         const float4 pa = a.L.rec[prev.light].a, pb = a.L.rec[prev.light].b;
@@ -681,8 +681,8 @@ __device__ __forceinline__ Merge spatial_merge(const FrameArgs& a, int x, int y)
 {
     Merge g;
     const size_t idx = (size_t)y * a.W + x;
-    const uint4 o0 = a.B.r0[idx];
-    g.res = res_from(o0, a.B.r1[idx], a.B.r2[idx]);
+    const uint4 o0 = a.B.rec[idx].r0;
+    g.res = res_from(o0, a.B.rec[idx].r1, a.B.r2[idx]);
     g.shadow = o0.x & (kTraced | kVisible);
     g.hitw = a.cur.hitw[idx];
     g.dist = __uint_as_float(o0.y);  // the hit buffer's distance, as the candidate pass recorded it
@@ -807,11 +807,11 @@ __device__ __forceinline__ float mis_weight_tile(const FrameArgs& a, int x, int 
             const int nx = x + dx, ny = y + dy;
             const size_t ni = (size_t)ny * a.W + nx;
             const uint32_t nh = a.cur.hitw[ni];
-            const uint4 n0 = a.B.r0[ni];
+            const uint4 n0 = a.B.rec[ni].r0;
             const Shading t = shading_at(a, nx, ny, nh, __uint_as_float(n0.y));
             float p = phat(a.point, res.pos, Nl, t.sp, t.N, t.brdf, f3{lb.x, lb.y, lb.z}, la.w);
             if (p > 0.0f) {
-                const int known = known_visibility(n0.x, a.B.r1[ni], res.light, res.pos);
+                const int known = known_visibility(n0.x, a.B.rec[ni].r1, res.light, res.pos);
                 if (known == 0) {
                     p = 0.0f;
                 } else if (known < 0) {
@@ -834,7 +834,7 @@ __device__ __forceinline__ float mis_weight_tile(const FrameArgs& a, int x, int 
             const float4 smp = L.sample[owner];
             const uint32_t light = __float_as_uint(smp.w);
             const int nx = (int)(ni % a.W), ny = (int)(ni / a.W);
-            const float nd = __uint_as_float(a.B.r0[ni].y);
+            const float nd = __uint_as_float(a.B.rec[ni].r0.y);
             const Shading sh = shading_at(a, nx, ny, a.cur.hitw[ni], nd);
             const f3 spo = f3{sh.sp.x + 0.1f * sh.N.x, sh.sp.y + 0.1f * sh.N.y, sh.sp.z + 0.1f * sh.N.z};
             const f3 Ld = normalize(sub(f3{smp.x, smp.y, smp.z}, spo));
@@ -910,10 +910,10 @@ __device__ __forceinline__ bool shade_px(const FrameArgs& a, int x, int y)
         }
         f3 add = f3{0.0f, 0.0f, 0.0f};
         if (a.gfxexp || !is_emitter(voxel)) {
-            const uint4 r0 = a.A.r0[idx];
+            const uint4 r0 = a.A.rec[idx].r0;
             const float W = __uint_as_float(r0.z);
             if (W > 0.0f && (r0.x & 0xffffffu) > 0u) {
-                const uint4 r1 = a.A.r1[idx];
+                const uint4 r1 = a.A.rec[idx].r1;
                 const uint32_t light = r1.w;
                 if (light < a.L.n) {
                     const f3 pos = f3{__uint_as_float(r1.x), __uint_as_float(r1.y), __uint_as_float(r1.z)};
@@ -940,7 +940,7 @@ __device__ __forceinline__ bool shade_px(const FrameArgs& a, int x, int y)
                         asm volatile("" : "+v"(h), "+v"(i2));
                         if (park) h = a.cur.hitw[i2];
                         const f3 sp = park ? f3{pp.x, pp.y, pp.z} : s.sp;
-                        const uint4 q0 = a.A.r0[i2], q1 = a.A.r1[i2];
+                        const uint4 q0 = a.A.rec[i2].r0, q1 = a.A.rec[i2].r1;
                         const float4 qa = a.L.rec[q1.w].a, qb = a.L.rec[q1.w].b;
                         const float Wq = __uint_as_float(q0.z), invPdf = __uint_as_float(q0.w);
                         const f3 posq = f3{__uint_as_float(q1.x), __uint_as_float(q1.y), __uint_as_float(q1.z)};
@@ -949,7 +949,7 @@ __device__ __forceinline__ bool shade_px(const FrameArgs& a, int x, int y)
                         add = f3{inc.x * Wq * invPdf, inc.y * Wq * invPdf, inc.z * Wq * invPdf};
                     } else {
                         // discard: W = wsum = 0 (ris.cl:276-281)
-                        reinterpret_cast<uint32_t*>(&a.A.r0[pidx])[2] = 0u;
+                        reinterpret_cast<uint32_t*>(&a.A.rec[pidx].r0)[2] = 0u;
                         reinterpret_cast<float*>(&a.A.r2[pidx])[0] = 0.0f;
                     }
                 }
@@ -1124,7 +1124,7 @@ __device__ __forceinline__ void resolve_tile(const FrameArgs& a, int x, int y)
             store_res(a.A, idx, g.res, g.hitw, g.dist, g.shadow);
         }
         const float W = mis_weight_tile<kNested>(a, x, y, g, in);
-        if (in && g.merged) a.A.r0[idx].z = __float_as_uint(W);
+        if (in && g.merged) a.A.rec[idx].r0.z = __float_as_uint(W);
     } else if (in) {
         spatial_px(a, x, y);
     }
@@ -1169,13 +1169,13 @@ __device__ __forceinline__ MisTap mis_tap(const FrameArgs& a, int x, int y, cons
     const int nx = x + dx, ny = y + dy;
     const size_t ni = (size_t)ny * a.W + nx;
     const uint32_t nh = a.cur.hitw[ni];
-    const uint4 n0 = a.B.r0[ni];
+    const uint4 n0 = a.B.rec[ni].r0;
     const Shading t = shading_at(a, nx, ny, nh, __uint_as_float(n0.y));
     MisTap o;
     o.p = phat(a.point, res.pos, Nl, t.sp, t.N, t.brdf, f3{lb.x, lb.y, lb.z}, la.w);
     o.ray = false;
     if (o.p > 0.0f) {
-        const int known = known_visibility(n0.x, a.B.r1[ni], res.light, res.pos);
+        const int known = known_visibility(n0.x, a.B.rec[ni].r1, res.light, res.pos);
         if (known == 0) o.p = 0.0f;
         o.ray = known < 0;
     }
@@ -1265,9 +1265,9 @@ struct MisRay {
 __device__ __forceinline__ MisRay mis_ray(const FrameArgs& a, uint2 task)
 {
     const uint32_t owner = task.x >> 5, ni = task.y;
-    const uint4 smp = a.A.r1[owner];
+    const uint4 smp = a.A.rec[owner].r1;
     const int nx = (int)(ni % a.W), ny = (int)(ni / a.W);
-    const float nd = __uint_as_float(a.B.r0[ni].y);
+    const float nd = __uint_as_float(a.B.rec[ni].r0.y);
     const Shading sh = shading_at(a, nx, ny, a.cur.hitw[ni], nd);
     MisRay r;
     r.spo = f3{sh.sp.x + 0.1f * sh.N.x, sh.sp.y + 0.1f * sh.N.y, sh.sp.z + 0.1f * sh.N.z};
@@ -1348,7 +1348,7 @@ __global__ __launch_bounds__(256) VR_WAVES(W) void k_mis_finish(FrameArgs a, Mis
             const int sel = (int)info.z - 1;
             float Wm = 0.0f;
             if (res.wsum > 0.0f && res.light < b.L.n) {
-                const float dist = __uint_as_float(b.A.r0[idx].y);
+                const float dist = __uint_as_float(b.A.rec[idx].r0.y);
                 const Shading s = shading_at(b, x, y, hitw, dist);
                 const float4 la = b.L.rec[res.light].a, lb = b.L.rec[res.light].b;
                 const f3 Nl = face_normal(res.face);
@@ -1368,7 +1368,7 @@ __global__ __launch_bounds__(256) VR_WAVES(W) void k_mis_finish(FrameArgs a, Mis
                 const float Wq = (res.wsum * psel) / d;
                 Wm = (d > 0.0f && isfinite(Wq)) ? Wq : 0.0f;
             }
-            b.A.r0[idx].z = __float_as_uint(Wm);
+            b.A.rec[idx].r0.z = __float_as_uint(Wm);
         }
     }
     shade_tile<false, kNested>(b, x, y, in);

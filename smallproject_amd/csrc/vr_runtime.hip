@@ -110,9 +110,8 @@ struct vr_ctx {
     float* dist[2] = {};
     uint32_t* seed[2] = {};
     // reservoir records (ResPlanes), [0] = A (final), [1] = B (initial +
-    // temporal): 16 + 16 + 8 bytes per pixel
-    uint4* rr0[2] = {};
-    uint4* rr1[2] = {};
+    // temporal): 32 + 8 bytes per pixel
+    Record* rec[2] = {};
     float2* rr2[2] = {};
     unsigned long long* rays = nullptr;  // [kRayKinds] traced-ray counters
     bool countRays = false;
@@ -369,8 +368,8 @@ FrameArgs frame_args(const vr_ctx* c, const vr_render_params* p)
     }
     const int cur = c->cur;
     a.cur = HitPlanes{c->hitw[cur], c->dist[cur], c->seed[cur]};
-    a.A = ResPlanes{c->rr0[0], c->rr1[0], c->rr2[0]};
-    a.B = ResPlanes{c->rr0[1], c->rr1[1], c->rr2[1]};
+    a.A = ResPlanes{c->rec[0], c->rr2[0]};
+    a.B = ResPlanes{c->rec[1], c->rr2[1]};
     a.rays = c->countRays ? c->rays : nullptr;
     a.frame = c->frame;
     a.emitLut = c->emitLut;
@@ -527,7 +526,7 @@ int vr_create(const vr_config* cfg, vr_ctx** out)
            ok(dalloc(&c->emitLut, 256)) && ok(dalloc(&c->frame, n)) && ok(dalloc(&c->rays, (size_t)kRayKinds));
     for (int i = 0; good && i < 2; i++)
         good = ok(dalloc(&c->hitw[i], n)) && ok(dalloc(&c->dist[i], n)) && ok(dalloc(&c->seed[i], n)) &&
-               ok(dalloc(&c->rr0[i], n)) && ok(dalloc(&c->rr1[i], n)) && ok(dalloc(&c->rr2[i], n));
+               ok(dalloc(&c->rec[i], n)) && ok(dalloc(&c->rr2[i], n));
     if (good) {
         good = ok(hipMemsetAsync(c->grid, 0, (size_t)VR_GRIDSIZE * 4, c->stream)) &&
                ok(hipMemsetAsync(c->uber, 0, 4096, c->stream)) &&
@@ -537,8 +536,9 @@ int vr_create(const vr_config* cfg, vr_ctx** out)
                ok(hipMemsetAsync(c->frame, 0, n * 16, c->stream));
         for (int i = 0; good && i < 2; i++)
             good = ok(hipMemsetAsync(c->hitw[i], 0, n * 4, c->stream)) && ok(hipMemsetAsync(c->dist[i], 0, n * 4, c->stream)) &&
-                   ok(hipMemsetAsync(c->seed[i], 0, n * 4, c->stream)) && ok(hipMemsetAsync(c->rr0[i], 0, n * 16, c->stream)) &&
-                   ok(hipMemsetAsync(c->rr1[i], 0, n * 16, c->stream)) && ok(hipMemsetAsync(c->rr2[i], 0, n * 8, c->stream));
+                   ok(hipMemsetAsync(c->seed[i], 0, n * 4, c->stream)) &&
+                   ok(hipMemsetAsync(c->rec[i], 0, n * sizeof(Record), c->stream)) &&
+                   ok(hipMemsetAsync(c->rr2[i], 0, n * 8, c->stream));
         good = good && ok(hipMemsetAsync(c->rays, 0, kRayKinds * 8, c->stream));
         good = good && ok(hipStreamSynchronize(c->stream));
     }
@@ -566,7 +566,7 @@ int vr_destroy(vr_ctx* c)
     dfree(c->rays);
     for (int i = 0; i < 2; i++) {
         dfree(c->hitw[i]), dfree(c->dist[i]), dfree(c->seed[i]);
-        dfree(c->rr0[i]), dfree(c->rr1[i]), dfree(c->rr2[i]);
+        dfree(c->rec[i]), dfree(c->rr2[i]);
     }
     dfree(c->mlpP), dfree(c->mlpM), dfree(c->mlpV), dfree(c->mlpG);
     dfree(c->mlpW1b), dfree(c->mlpW2b), dfree(c->mlpW2Tb), dfree(c->mlpW3b), dfree(c->mlpW3Tb);
@@ -857,21 +857,21 @@ int vr_read_reservoirs(vr_ctx* c, int which, float* a4, float* b4, uint32_t* m)
     const size_t n = (size_t)c->cfg.width * c->cfg.height;
     HIPCHK(c, hipStreamSynchronize(c->stream));
     // the records (ResPlanes) rearranged into the documented planes
-    std::vector<uint4> r0(n), r1(n);
+    std::vector<Record> rec(n);
     std::vector<float2> r2(n);
-    HIPCHK(c, hipMemcpy(r0.data(), c->rr0[which], n * 16, hipMemcpyDeviceToHost));
-    HIPCHK(c, hipMemcpy(r1.data(), c->rr1[which], n * 16, hipMemcpyDeviceToHost));
+    HIPCHK(c, hipMemcpy(rec.data(), c->rec[which], n * sizeof(Record), hipMemcpyDeviceToHost));
     HIPCHK(c, hipMemcpy(r2.data(), c->rr2[which], n * 8, hipMemcpyDeviceToHost));
     for (size_t i = 0; i < n; i++) {
+        const uint4 r0 = rec[i].r0, r1 = rec[i].r1;
         if (a4) {
-            a4[4 * i + 0] = r2[i].x, a4[4 * i + 1] = bits_float(r0[i].z);
-            a4[4 * i + 2] = r2[i].y, a4[4 * i + 3] = bits_float(r0[i].w);
+            a4[4 * i + 0] = r2[i].x, a4[4 * i + 1] = bits_float(r0.z);
+            a4[4 * i + 2] = r2[i].y, a4[4 * i + 3] = bits_float(r0.w);
         }
         if (b4) {
-            b4[4 * i + 0] = bits_float(r1[i].x), b4[4 * i + 1] = bits_float(r1[i].y);
-            b4[4 * i + 2] = bits_float(r1[i].z), b4[4 * i + 3] = bits_float(r1[i].w);
+            b4[4 * i + 0] = bits_float(r1.x), b4[4 * i + 1] = bits_float(r1.y);
+            b4[4 * i + 2] = bits_float(r1.z), b4[4 * i + 3] = bits_float(r1.w);
         }
-        if (m) m[i] = r0[i].x & 0x07ffffffu;  // M | face << 24
+        if (m) m[i] = r0.x & 0x07ffffffu;  // M | face << 24
     }
     return VR_OK;
 }
