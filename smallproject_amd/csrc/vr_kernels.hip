@@ -671,12 +671,29 @@ struct Merge {
     Res res;
     Shading s;
     uint32_t hitw, seed, seed0, M0, mask, shadow;
+    uint32_t seedKept;  // kKeep: the stream before tap kTapsKept
     float dist;
     int sel;
     bool merged;
 };
 
-template <bool kMis>
+// The pixels of a thread's first combined taps, kept in LDS: finding one again
+// from the stream costs a sine and a cosine (k_mis_list found them twice more;
+// 5 taps at 1279x717: 203 -> 193 us, with the shorter sine).  8 taps fit
+// beside 8 waves per SIMD; later ones are found again.
+constexpr uint32_t kTapsKept = 8u;
+
+struct TapLds {
+    uint32_t px[kTapsKept][256];
+};
+
+__device__ __forceinline__ TapLds& tap_lds()
+{
+    __shared__ TapLds l;
+    return l;
+}
+
+template <bool kMis, bool kKeep = false>
 __device__ __forceinline__ Merge spatial_merge(const FrameArgs& a, int x, int y)
 {
     Merge g;
@@ -686,7 +703,7 @@ __device__ __forceinline__ Merge spatial_merge(const FrameArgs& a, int x, int y)
     g.shadow = o0.x & (kTraced | kVisible);
     g.hitw = a.cur.hitw[idx];
     g.dist = __uint_as_float(o0.y);  // the hit buffer's distance, as the candidate pass recorded it
-    g.mask = 0u, g.sel = -1;
+    g.mask = 0u, g.sel = -1, g.seedKept = 0u;
     g.merged = (g.hitw & 0xffffffu) != 0u && a.spatial;
     if (!g.merged) return g;
     Res& res = g.res;
@@ -697,6 +714,7 @@ __device__ __forceinline__ Merge spatial_merge(const FrameArgs& a, int x, int y)
     const Shading& s = g.s;
     const float rad = (float)(a.spatialRadius - 1u);
     for (uint32_t i = 0; i < a.spatialTaps; i++) {
+        if (kKeep && i == kTapsKept) g.seedKept = seed;
         int dx, dy;
         tap_offset(seed, rad, dx, dy);
         const int nx = x + dx, ny = y + dy;
@@ -722,6 +740,7 @@ __device__ __forceinline__ Merge spatial_merge(const FrameArgs& a, int x, int y)
             g.shadow = 0u;
         }
         if (kMis) g.mask |= 1u << i;
+        if (kKeep && i < kTapsKept) tap_lds().px[i][threadIdx.x] = (uint32_t)ni;
     }
     res_adjust(res, res.pHat);
     g.seed = seed;
@@ -1152,22 +1171,16 @@ __global__ __launch_bounds__(256) VR_WAVES(W) void k_resolve(FrameArgs a)
 // Combined tap i of a pixel's MIS weight for its merged sample (res, with
 // the sample's face normal Nl and light records la, lb): the neighbour's
 // target T (0 when the candidate pass found the sample occluded from there),
-// whether a ray must decide its visibility, its pixel and its M.  `rs` is
-// the replayed stream at tap i's offset draws.
+// whether a ray must decide its visibility, and its M.
 struct MisTap {
     float p;
     bool ray;
-    uint32_t ni, M;
+    uint32_t M;
 };
 
-__device__ __forceinline__ MisTap mis_tap(const FrameArgs& a, int x, int y, const Res& res, f3 Nl, float4 la,
-                                          float4 lb, uint32_t& rs, float rad)
+__device__ __forceinline__ MisTap mis_tap(const FrameArgs& a, uint32_t ni, const Res& res, f3 Nl, float4 la, float4 lb)
 {
-    int dx, dy;
-    tap_offset(rs, rad, dx, dy);
-    (void)rnd(rs);  // the merge's draw
-    const int nx = x + dx, ny = y + dy;
-    const size_t ni = (size_t)ny * a.W + nx;
+    const int nx = (int)(ni % a.W), ny = (int)(ni / a.W);
     const uint32_t nh = a.cur.hitw[ni];
     const uint4 n0 = a.B.rec[ni].r0;
     const Shading t = shading_at(a, nx, ny, nh, __uint_as_float(n0.y));
@@ -1179,16 +1192,20 @@ __device__ __forceinline__ MisTap mis_tap(const FrameArgs& a, int x, int y, cons
         if (known == 0) o.p = 0.0f;
         o.ray = known < 0;
     }
-    o.ni = (uint32_t)ni;
     o.M = n0.x & 0xffffffu;
     return o;
 }
 
-// skip tap i's offset draws (a tap that was not combined)
-__device__ __forceinline__ void mis_skip_tap(uint32_t& rs, float rad)
+// Pixel of tap i, a combined one or not (then it draws no merge number and
+// the value does not count); `rs`: seedKept, carried from tap to tap.
+__device__ __forceinline__ uint32_t tap_pixel(const FrameArgs& a, int x, int y, uint32_t i, bool combined, uint32_t& rs,
+                                              float rad)
 {
+    if (i < kTapsKept) return tap_lds().px[i][threadIdx.x];
     int dx, dy;
     tap_offset(rs, rad, dx, dy);
+    if (combined) (void)rnd(rs);
+    return (uint32_t)((y + dy) * (int)a.W + (x + dx));
 }
 
 template <int W>
@@ -1205,7 +1222,7 @@ __global__ __launch_bounds__(256) VR_WAVES(W) void k_mis_list(FrameArgs a, MisBu
     f3 Nl = f3{0.0f, 0.0f, 0.0f};
     bool need = false;
     if (in) {
-        g = spatial_merge<true>(a, x, y);
+        g = spatial_merge<true, true>(a, x, y);
         if (g.merged) a.cur.seed[idx] = g.seed;
         store_res(a.A, idx, g.res, g.hitw, g.dist, g.shadow);  // W: k_mis_finish
         m.occ[idx] = 0u;
@@ -1214,13 +1231,12 @@ __global__ __launch_bounds__(256) VR_WAVES(W) void k_mis_list(FrameArgs a, MisBu
             la = a.L.rec[g.res.light].a, lb = a.L.rec[g.res.light].b;
             Nl = face_normal(g.res.face);
             const size_t npx = (size_t)a.W * a.H;
-            uint32_t rs = g.seed0;
+            uint32_t rs = g.seedKept;
             for (uint32_t i = 0; i < a.spatialTaps && (g.mask >> i); i++) {
-                if (!((g.mask >> i) & 1u)) {
-                    mis_skip_tap(rs, rad);
-                    continue;
-                }
-                const MisTap t = mis_tap(a, x, y, g.res, Nl, la, lb, rs, rad);
+                const bool combined = ((g.mask >> i) & 1u) != 0u;
+                const uint32_t ni = tap_pixel(a, x, y, i, combined, rs, rad);
+                if (!combined) continue;
+                const MisTap t = mis_tap(a, ni, g.res, Nl, la, lb);
                 // the term as the one-kernel merge adds it, (float)M * T
                 m.terms[i * npx + idx] = make_float2((float)t.M * t.p, t.p);
                 if (t.ray) rays |= 1u << i;
@@ -1241,16 +1257,11 @@ __global__ __launch_bounds__(256) VR_WAVES(W) void k_mis_list(FrameArgs a, MisBu
     if (lane == 63u && total != 0u) base = atomicAdd(m.count, total);
     base = __shfl(base, 63, 64);
     if (rays != 0u) {
-        // replay the offsets of the listed taps
         uint32_t slot = base + incl - n;
-        uint32_t rs = g.seed0;
+        uint32_t rs = g.seedKept;
         for (uint32_t i = 0; i < a.spatialTaps && (rays >> i); i++) {
-            int dx, dy;
-            tap_offset(rs, rad, dx, dy);
-            if (!((g.mask >> i) & 1u)) continue;
-            (void)rnd(rs);
-            if ((rays >> i) & 1u)
-                m.list[slot++] = make_uint2(((uint32_t)idx << 5) | i, (uint32_t)((size_t)(y + dy) * a.W + (x + dx)));
+            const uint32_t ni = tap_pixel(a, x, y, i, ((g.mask >> i) & 1u) != 0u, rs, rad);
+            if ((rays >> i) & 1u) m.list[slot++] = make_uint2(((uint32_t)idx << 5) | i, ni);
         }
     }
 }
@@ -1558,6 +1569,7 @@ __global__ __launch_bounds__(256) VR_WAVES(5) void k_ground_truth(FrameArgs a, u
                     const float sinTheta = sqrtf(1 - r0 * r0);
                     float sn, cs;
                     sincos_det(kTwoPi * r1, sn, cs);
+                    asm volatile("" : "+v"(sn), "+v"(cs));  // before the hit's vectors are read back: fewer registers
                     const float xs = sinTheta * cs, zs = sinTheta * sn;
                     const float4 O2 = vload(g.O[lane]), N = vload(g.N[lane]), Nt = vload(g.T[lane]), Nb = vload(g.B[lane]);
                     const f3 R = f3{xs * Nb.x + r0 * N.x + zs * Nt.x, xs * Nb.y + r0 * N.y + zs * Nt.y,
