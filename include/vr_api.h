@@ -257,10 +257,11 @@ int vr_read_frame(vr_ctx* ctx, float* rgba);
 
 /* Per-stage device time of the last rendered frame, milliseconds, measured
  * with HIP events around each stage (template/world.cpp:2439-2471).  When
- * the context is the only one in the process and nothing changed the world
- * since the previous frame's candidate pass, the primary pass runs on a
- * second stream beside that frame's last stage; its time then spans its run
- * next to that stage. */
+ * the context also rendered the process's previous frame, that frame has not
+ * ended and nothing changed the world since its candidate pass, the primary
+ * pass runs on a second stream beside that frame's later stages (frames of
+ * up to 655,360 pixels) or its last one; its time then spans its run next to
+ * them. */
 int vr_stage_times(vr_ctx* ctx, float ms[VR_NUM_STAGES]);
 
 /* Rays traced by the following frames (a diagnostic with no counterpart in

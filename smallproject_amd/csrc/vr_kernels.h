@@ -121,7 +121,7 @@ __device__ __forceinline__ void tile_of_block(uint32_t order, int& tx, int& ty)
 }
 
 // traversal of a stage's shadow rays (FrameArgs::dda; the values of
-// VR_DDA_SCHEDULED and VR_DDA_NESTED): the wave-scheduled walk, or the
+// VR_DDA_SCHEDULED and VR_DDA_NESTED): the unified walk, or the
 // nested one of the primary rays
 constexpr uint32_t kDdaScheduled = 0u, kDdaNested = 1u;
 

@@ -23,12 +23,14 @@ using namespace vr;
 
 static constexpr int kRing = 64;  // frames whose stage events are kept
 
-// contexts alive in the process: a context overlaps its own frames (below)
-// only while it is the only one.  With several, their streams already
+// The context (by number) that queued the process's last frame: a context
+// overlaps its own frames (below) while it renders frame after frame, whatever
+// other contexts are alive.  When contexts take turns, their streams already
 // overlap each other's work, and a second stream each would crowd the
 // process's few hardware queues (measured: 16 Worlds rendered view after
-// view, 6.7 -> 8.3 ms per round).
-static std::atomic<int> g_liveContexts{0};
+// view, 6.7 -> 8.3 ms per round).  It decides where a pass is queued, never
+// what it computes.
+static std::atomic<uint64_t> g_contexts{0}, g_lastFrame{0};
 
 // Scratch of vr_trace_rays_noalloc: VR_NOALLOC_MAX_RAYS rays and their hits
 // staged on the device (origins and directions 12 B each, voxel, distance and
@@ -70,13 +72,20 @@ struct vr_ctx {
     void* scratch = nullptr;
     hipError_t noScratch = hipSuccess;
     // The next frame's primary pass may run on `side` beside this frame's
-    // spatial reuse + shading: it writes the hit buffer that only this
-    // frame's candidate pass read (`initDone`), unless work queued since then
-    // changed the world it traces (`worldEpoch`, advanced by vr_scene_step;
-    // vr_commit returns only once its uploads are done).  `side` is created
-    // on first use.
+    // later passes: it writes the other hit buffer, last read by the frame
+    // before this one, whose passes end before this frame's candidate pass
+    // starts (its stage's start event), unless work queued since then changed
+    // the world it traces (`worldEpoch`, advanced by vr_scene_step; vr_commit
+    // returns only once its uploads are done).  `side` is created on first
+    // use.
+    //   A small frame (kSmallFrame) lets the next primary pass start beside
+    // its candidate pass, whose last waves leave much of the chip idle; in a
+    // large one both are bound by instruction issue, and the primary pass
+    // waits for the candidates' end (`initDone`) to run beside the last
+    // stage, which waits for memory.  So it does with the learned source,
+    // whose proposal follows it on `side`.
     hipStream_t side = nullptr;
-    bool counted = false;  // included in g_liveContexts
+    uint64_t number = 0;  // 1, 2, ... in the order of creation
     hipEvent_t initDone = nullptr, primDone = nullptr;
     // The learned proposal follows the primary pass on `side` too; it reads
     // the network's weights as of their last update, recorded here on
@@ -549,8 +558,7 @@ int vr_create(const vr_config* cfg, vr_ctx** out)
     // set-up of the allocation-free entry point, with the context's device
     // current: a failed lookup leaves every other entry point working
     c->scratch = scratch_address(c->device, &c->noScratch);
-    g_liveContexts++;
-    c->counted = true;
+    c->number = ++g_contexts;
     *out = c;
     return VR_OK;
 }
@@ -558,7 +566,6 @@ int vr_create(const vr_config* cfg, vr_ctx** out)
 int vr_destroy(vr_ctx* c)
 {
     if (!c) return VR_ERR_ARG;
-    if (c->counted) g_liveContexts--;
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     if (c->side) (void)hipStreamSynchronize(c->side);
     dfree(c->grid), dfree(c->uber), dfree(c->bricks), dfree(c->proj), dfree(c->stageIds), dfree(c->stageData);
@@ -727,6 +734,14 @@ static int mis_alloc(vr_ctx* c, uint32_t taps, bool& mis_split)
     return VR_OK;
 }
 
+// Frames of up to this many pixels let the next frame's primary pass start
+// beside their candidate pass (the other way in brackets, whole frames): 10
+// waves of it a SIMD, 6 of them at a time.  601x347 behind panes, whose
+// primary pass is as long as its longest wave, 2.58 (3.35) ms for 8; 960x540
+// area 7.5 (8.0), point lights 2.48 (2.56); 1279x717 power + MIS 14.6 (14.4);
+// 1920x1080 area 20.0 (19.4).
+static constexpr size_t kSmallFrame = (size_t)256 * 4 * 10 * 64;
+
 int vr_render_frame(vr_ctx* c, const vr_render_params* p)
 {
     if (!c || !p) return VR_ERR_ARG;
@@ -749,15 +764,26 @@ int vr_render_frame(vr_ctx* c, const vr_render_params* p)
     }
     c->cur = 1 - c->cur;  // primaryHitBuffer swap, world.cpp:2221-2223
     const FrameArgs a = frame_args(c, p);
-    // the primary pass beside the previous frame's last stage when nothing
-    // since that frame's candidate pass has changed the world
-    bool overlap = c->initRecorded && c->epochAtInit == c->worldEpoch && g_liveContexts.load() == 1;
+    // the primary pass beside the previous frame's later stages when nothing
+    // since that frame's candidate pass was queued has changed the world
+    const bool again = g_lastFrame.exchange(c->number) == c->number;
+    bool overlap = again && c->initRecorded && c->lastSlot >= 0 && c->epochAtInit == c->worldEpoch;
+    if (overlap && hipEventQuery(c->ev[c->lastSlot][2 * VR_NUM_STAGES - 1]) == hipSuccess) {
+        // that frame has ended: there is nothing to run beside, and a pass on
+        // the second stream starts later (320x180, one frame a read-back:
+        // 322 us with it, 315 without)
+        overlap = false;
+    } else if (overlap) {
+        (void)hipGetLastError();  // "not ready" is no error of a later launch
+    }
     if (overlap && !c->side && hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking) != hipSuccess) {
         c->side = nullptr;
         overlap = false;
     }
     hipStream_t ps = overlap ? c->side : c->stream;
-    if (overlap) HIPCHK(c, hipStreamWaitEvent(c->side, c->initDone, 0));
+    const bool early = !learned && (size_t)c->cfg.width * c->cfg.height <= kSmallFrame;
+    if (overlap)
+        HIPCHK(c, hipStreamWaitEvent(c->side, early ? c->ev[c->lastSlot][2 * VR_STAGE_INITIAL] : c->initDone, 0));
     for (int s = 0; s < VR_NUM_STAGES; s++) {
         FrameArgs as = a;
         as.tileOrder = (c->cfg.flags >> (2 * s)) & 3u;
@@ -789,7 +815,7 @@ int vr_render_frame(vr_ctx* c, const vr_render_params* p)
         }
         HIPCHK(c, hipEventRecord(c->ev[slot][2 * s + 1], st));
         if (s == VR_STAGE_INITIAL) {
-            HIPCHK(c, hipEventRecord(c->initDone, c->stream));
+            if (!early) HIPCHK(c, hipEventRecord(c->initDone, c->stream));
             c->initRecorded = true;
             c->epochAtInit = c->worldEpoch;
         }
@@ -1249,6 +1275,11 @@ int vr_mlp_train(vr_ctx* c, const vr_ctx* from, uint32_t nsamples, float lr, uin
     a.L.n = src->nLights;
     HIPCHK(c, launch_train_gather(a, c->clusterOf, nsamples, (uint32_t)src->frameNo * 0x9e3779b9u + 0x7f4a7c15u,
                                   c->trainX, c->trainT, c->trainW, c->stream));
+    if (src != c) {
+        // the sample context's next passes overwrite what the gather reads
+        HIPCHK(c, hipEventRecord(c->weightsReady, c->stream));
+        HIPCHK(c, hipStreamWaitEvent(src->stream, c->weightsReady, 0));
+    }
     // `steps` minibatches of consecutive samples (each spread over the image)
     const uint32_t nb = steps < nsamples ? steps : nsamples;
     for (uint32_t s = 0; s < nb; s++) {
